@@ -3,8 +3,8 @@
 // decoding model's projections (F.linear on wqkv, wo, gate_up_proj, down_proj and the lm head,
 // models/llama.py:192,203,208,214 and the lm head at models/base.py:98).
 //
-// At M <= 16 the call is bound by reading the weight once from HBM (2*N*K bytes), so the kernel
-// is laid out for the load path, not for the matrix cores: every wave load reads 1 KB of ONE
+// At M <= 16 the call is bound by reading the weight once from HBM (2*N*K bytes), so the kernels
+// are laid out for the load path. Up to 4 token rows (linear_kernel): every wave load reads 1 KB of ONE
 // weight row (64 lanes x 16 B, fully coalesced), and the arithmetic runs on the VALU as bf16 dot2
 // with fp32 accumulation (v_dot2c_f32_bf16), which needs no operand shuffles. A workgroup owns R
 // weight rows; its waves split K into 512-element blocks (wave w takes blocks w, w+nw, ...) with
@@ -13,13 +13,15 @@
 // lane holds), then summed across rows and waves in LDS; one rounding to bf16 at the end.
 //
 // The QKV projection with the new token's RoPE and KV append in its epilogue
-// (skv_linear_qkv_rope_append): a workgroup's 8 output rows lie in one head, and with the
+// (skv_linear_qkv_rope_append): a workgroup's 8 or 16 output rows lie in one head, and with the
 // half-split heads' q/k weight rows interleaved (dims d and d + 64 adjacent; GLM's rotation pairs
 // are adjacent already) every rotation pair of the workgroup is in it. The workgroup rounds its
 // sums to bf16, rotates them with the bf16 per-op rounding of skv_rope_qk_append and writes q to
 // q_out and k, v to the append row of the key/value buffers: bit-identical to skv_linear followed
 // by skv_rope_qk_append, one launch and the fused row's round trip fewer. The position and
 // cos/sin loads are issued before the weight stream starts.
+#include <type_traits>
+
 #include "rope_math.h"
 #include "skv_common.h"
 
@@ -275,6 +277,172 @@ __global__ void __launch_bounds__(kMaxWaves * 64) linear_kernel(const uint16_t* 
   }
 }
 
+
+// The matrix-core form, for 5 to 16 token rows. Bound: the weight stream from HBM. The dot2 form
+// above needs R * MP accumulators and re-reads x once per R weight rows, so at 9..16 rows, where
+// registers leave R = 2, its x traffic from the L2 is eight times the weight stream and bounds it.
+// Here a workgroup owns 16 weight rows (one 16x16 MFMA tile; 8 of a small weight, for twice the
+// workgroups) and its waves split K into 128-element
+// blocks (wave w takes blocks w, w + NW, ...). A wave reads its block of the weight and x rows with
+// whole 256-byte row segments per load (the MFMA operand order read directly from memory, 64 bytes
+// of 16 rows a load, streamed at 4.1 against 5.6 TB/s), puts it into its own LDS tile (16-byte
+// chunk q of row r at slot q ^ r: reads and writes without bank conflicts, no barrier), requests
+// the next block and reads the tile back in operand order (A = weight rows, B = token rows). The
+// waves' sums are added in wave order at the end and finished in pairs of weight rows.
+// MI355X, cold weights, gate/up 28672 x 4096: 16 rows 122 -> 42 us, 8 rows 45.2 -> 37.4 us
+// (6.3 TB/s); down 4096 x 14336: 58 -> 23.4 us, 24.1 -> 21.9 us; head 128256 x 4096 at 8 rows:
+// 174 -> 154 us.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kTileK = 128;                 // k elements per block
+constexpr int kTileChunks = kTileK / 8;     // 16-byte chunks per tile row
+constexpr int kLoadRows = 64 / kTileChunks; // tile rows per wave load
+
+// RW: weight rows of the workgroup, MP: token rows of the x tile (8 or 16 each); NW: waves.
+template <int RW, int MP, int NW, bool kAct, int kRope>
+__global__ void __launch_bounds__(NW * 64) linear_mfma_kernel(const uint16_t* __restrict__ x, int64_t xs,
+                                                              const uint16_t* __restrict__ w, int64_t ws,
+                                                              uint16_t* __restrict__ y, int64_t ys, int M, int N,
+                                                              int K, RopeEpi re) {
+  static_assert(MP == 8 || MP == 16, "x tiles of 8 or 16 rows");
+  static_assert(RW == 8 || RW == 16, "weight tiles of 8 or 16 rows");
+  static_assert(!kAct || kRope == kNoRope, "one epilogue at a time");
+  constexpr int kWaveTile = (RW + MP) * kTileChunks;  // 16-byte chunks
+  constexpr int kLd = 17;                                    // padded row of the partial sums
+  static_assert(kWaveTile * 16 >= RW * kLd * 4, "the partial sums reuse the wave's tile");
+  __shared__ u32x4 tiles[NW * kWaveTile];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, grp = lane >> 4;
+  const int n0 = blockIdx.x * RW;
+
+  // The pair this thread finishes: weight rows n1, n1 + 1 of token row em (consecutive threads take
+  // consecutive pairs). Bias, position and append row are requested up front, cos/sin after the
+  // first weight block (so the wait for the position leaves the weight loads in flight).
+  const int ep = threadIdx.x % (RW / 2), em = threadIdx.x / (RW / 2);
+  const int n1 = n0 + 2 * ep;
+  const bool live = em < M && n1 < N;
+  float bias0 = 0.f, bias1 = 0.f;
+  if (re.bias && live) {
+    bias0 = skv::bf2f(re.bias[n1]);
+    bias1 = skv::bf2f(re.bias[min(n1 + 1, N - 1)]);
+  }
+  int64_t rp_pos = -1, rp_row = -1;
+  uint16_t rp_c = 0, rp_s = 0;
+  if constexpr (kRope != kNoRope) {
+    if (live) {
+      rp_pos = re.pos[em];
+      rp_row = *re.row_dev;
+    }
+  }
+
+  constexpr int kWl = RW / kLoadRows, kXl = MP / kLoadRows;  // wave loads per tile
+  u32x4* wt = tiles + wave * kWaveTile;
+  u32x4* xt = wt + RW * kTileChunks;
+  const int lrow = lane / kTileChunks, lq = lane % kTileChunks;
+  const char* wr[kWl];
+#pragma unroll
+  for (int i = 0; i < kWl; ++i)
+    wr[i] = reinterpret_cast<const char*>(w + static_cast<int64_t>(min(n0 + i * kLoadRows + lrow, N - 1)) * ws);
+  const char* xr[kXl];
+#pragma unroll
+  for (int i = 0; i < kXl; ++i)
+    xr[i] = reinterpret_cast<const char*>(x + static_cast<int64_t>(min(i * kLoadRows + lrow, M - 1)) * xs);
+  u32x4 wv[kWl], xv[kXl];
+  // A chunk past K (only in a last, partial block) is read at the row's start and stored as zeros.
+  auto load = [&](int b) {
+    const int k = b * kTileK + 8 * lq;
+    const uint32_t off = 2u * static_cast<uint32_t>(k < K ? k : 0);
+#pragma unroll
+    for (int i = 0; i < kWl; ++i) wv[i] = skv::load_nt(reinterpret_cast<const u32x4*>(wr[i] + off));
+#pragma unroll
+    for (int i = 0; i < kXl; ++i) xv[i] = *reinterpret_cast<const u32x4*>(xr[i] + off);
+    __builtin_amdgcn_sched_barrier(0);  // keep the loads ahead of the products that follow
+  };
+  const int nblk = (K + kTileK - 1) / kTileK;
+  if (wave < nblk) load(wave);
+  if constexpr (kRope != kNoRope) {
+    if (live) {
+      int head, d1, d2, kind, ci;
+      rope_pair_dims<kRope>(re, n1, head, d1, d2, kind, ci);
+      if (ci >= 0 && rp_pos >= 0 && rp_pos < re.cs_rows) {
+        const uint16_t* c = re.cs + rp_pos * re.cs_stride;
+        rp_c = c[ci];
+        rp_s = c[ci + (kRope == kRopeHalf ? 64 : 32)];
+      }
+    }
+  }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int b = wave; b < nblk; b += NW) {
+    const bool ok = b * kTileK + 8 * lq < K;
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < kWl; ++i) {
+      const int r = i * kLoadRows + lrow;
+      wt[r * kTileChunks + (lq ^ r)] = ok ? wv[i] : zero;
+    }
+#pragma unroll
+    for (int i = 0; i < kXl; ++i) {
+      const int r = i * kLoadRows + lrow;
+      xt[r * kTileChunks + (lq ^ r)] = ok ? xv[i] : zero;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (b + NW < nblk) load(b + NW);
+    const int wrow = li & (RW - 1), xrow = li & (MP - 1);  // (8-row tiles repeat, unused, in rows 8..15)
+#pragma unroll
+    for (int c = 0; c < kTileK / 32; ++c)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          __builtin_bit_cast(bf16x8, wt[wrow * kTileChunks + ((4 * c + grp) ^ wrow)]),
+          __builtin_bit_cast(bf16x8, xt[xrow * kTileChunks + ((4 * c + grp) ^ xrow)]), acc, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);  // the next block's writes stay behind these reads
+  }
+
+  // acc: lane (li, grp) holds weight rows 4*grp + r of token row li; summed over the waves, in wave
+  // order, by the thread of each pair.
+  float* red = reinterpret_cast<float*>(wt);  // (the wave's own tile)
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (RW == 16 || grp < 2) red[(4 * grp + r) * kLd + li] = acc[r];
+  __syncthreads();
+  if (!live) return;
+  float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    const float* p = reinterpret_cast<const float*>(tiles + i * kWaveTile) + 2 * ep * kLd + em;
+    s0 += p[0];
+    s1 += p[kLd];
+  }
+  if (re.bias) {  // (uniform: without a bias no add, so -0 sums stay -0)
+    s0 += bias0;
+    s1 += bias1;
+  }
+  if constexpr (kRope != kNoRope) {
+    int head, d1, d2, kind, ci;
+    rope_pair_dims<kRope>(re, n1, head, d1, d2, kind, ci);
+    const uint16_t x1 = skv::f2bf(s0), x2 = skv::f2bf(s1);
+    uint16_t y1 = x1, y2 = x2;
+    if (ci >= 0 && rp_pos >= 0 && rp_pos < re.cs_rows) skv::rope_half_split(x1, x2, rp_c, rp_s, y1, y2);
+    uint16_t* dst = nullptr;
+    if (kind == 0) {
+      dst = re.q_out + em * re.qo_sb + static_cast<int64_t>(head) * kHeadDim;
+    } else if (rp_row >= 0 && rp_row < re.buf_len) {  // beyond the buffer: nothing appended
+      const int h = kind == 1 ? head - re.Hq : head - re.Hq - re.Hkv;
+      dst = (kind == 1 ? re.k_cache : re.v_cache) + em * re.kv_sb + h * re.kv_sh + rp_row * re.kv_ss;
+    }
+    if (dst) {
+      dst[d1] = y1;
+      dst[d2] = y2;
+    }
+  } else if constexpr (kAct) {  // gate row n1, up row n1 + 1 (N is even)
+    y[static_cast<int64_t>(em) * ys + n1 / 2] = skv::f2bf(skv::silu_mul(skv::bround(s0), skv::bround(s1)));
+  } else {
+    uint16_t* dst = y + static_cast<int64_t>(em) * ys + n1;
+    dst[0] = skv::f2bf(s0);
+    if (n1 + 1 < N) dst[1] = skv::f2bf(s1);
+  }
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 int g_waves_override = -1;  // SKV_LINEAR_WAVES, read once
@@ -285,14 +453,40 @@ void launch(const uint16_t* x, int64_t xs, const uint16_t* w, int64_t ws, uint16
   const int groups = (N + R - 1) / R;
   const int nblk = (K + kBlockK - 1) / kBlockK;
   // Waves per workgroup, from sweeps of the Llama-3-8B projections and lm head on MI355X with
-  // cold weights: at up to 4 rows four waves win on every shape; at 8 rows (twice the
-  // registers, half the resident waves) four win on the 4096-row weights, one on wider ones,
-  // two on the vocabulary-sized head. At most one wave per k block.
-  int nw = MP <= 4 ? 4 : groups <= 512 ? 4 : groups >= 8192 ? 2 : 1;
+  // cold weights: four waves win on every shape. At most one wave per k block.
+  int nw = 4;
   if (g_waves_override > 0) nw = g_waves_override;
   while (nw > 1 && nw > nblk) nw /= 2;
   hipLaunchKernelGGL((linear_kernel<R, MP, kGated, kAct, kRope>), dim3(groups), dim3(64 * nw), 0, s, x, xs, w, ws, y,
                      ys, M, N, K, re);
+}
+
+
+// Tile rows and waves of the matrix-core form by the weight's rows (MI355X, cold weights, us at 8 / 16
+// token rows, K = 4096 where not given):
+//   n <= 2048: 8-row tiles, 16 waves, since 16-row tiles leave half of the 256 CUs idle (1000 x 16000:
+//     12.3 / 16.4 against 16.4 / 19.6 with 16-row tiles and 8 waves; 2048 x 4096: 5.9 / 6.9 against
+//     6.7 / 7.4); from n = 3072 on 16-row tiles win (7.2 / 7.9 against 7.9 / 11.2);
+//   4096 < n <= 8192, one to two workgroups per CU: 4 waves (6144: 11.1 / 12.7 against 11.9 / 13.2
+//     with 8; 8192: 12.7 / 13.8 against 13.0 / 14.2);
+//   else 8 waves (4096: 8.2 / 9.0 against 9.5 / 10.1 with 4 and 8.3 / 9.2 with 16; 4096 x 14336: 21.3 /
+//     23.4 against 26.4 / 27.8; 28672: 37.6 / 41.6 against 40.5 / 42.1).
+template <bool kAct, int kRope>
+void launch_mfma(const uint16_t* x, int64_t xs, const uint16_t* w, int64_t ws, uint16_t* y, int64_t ys, int M, int N,
+                 int K, hipStream_t s, const RopeEpi& re) {
+  auto go = [&](auto rw, auto mp, auto nw) {
+    constexpr int RW = decltype(rw)::value, MP = decltype(mp)::value, NW = decltype(nw)::value;
+    hipLaunchKernelGGL((linear_mfma_kernel<RW, MP, NW, kAct, kRope>), dim3((N + RW - 1) / RW), dim3(64 * NW), 0, s, x,
+                       xs, w, ws, y, ys, M, N, K, re);
+  };
+  auto rows = [&](auto mp) {
+    using std::integral_constant;
+    if (N <= 2048) go(integral_constant<int, 8>{}, mp, integral_constant<int, 16>{});
+    else if (N > 4096 && N <= 8192) go(integral_constant<int, 16>{}, mp, integral_constant<int, 4>{});
+    else go(integral_constant<int, 16>{}, mp, integral_constant<int, 8>{});
+  };
+  if (M <= 8) rows(std::integral_constant<int, 8>{});
+  else rows(std::integral_constant<int, 16>{});
 }
 
 template <bool kGated, bool kAct = false>
@@ -302,8 +496,8 @@ int linear_impl(const char* what, const uint16_t* x, int64_t x_stride, const uin
     skv_set_error("%s: null pointer", what);
     return SKV_EINVAL;
   }
-  // The gated form recomputes the activations of its rows in every workgroup, and its 8- and
-  // 16-row variants would hold two more sets of x registers: it is offered up to 4 rows only.
+  // The gated form recomputes the activations of its rows in every workgroup: it is offered up to
+  // 4 rows only.
   constexpr int kMaxRows = kGated ? 4 : 16;
   if (m < 1 || m > kMaxRows || n < 1 || k < 8 || k % 8) {
     skv_set_error("%s: m=%d n=%d k=%d (1 <= m <= %d, k a multiple of 8)", what, m, n, k, kMaxRows);
@@ -328,17 +522,17 @@ int linear_impl(const char* what, const uint16_t* x, int64_t x_stride, const uin
   const hipStream_t s = static_cast<hipStream_t>(stream);
   RopeEpi re{};
   re.bias = bias;
-  if (m == 1)
+  // The dot2 form up to 4 rows: at 4 it streams as fast as the matrix cores (28672 x 4096: 36.5 against
+  // 37.3 us, 6144 x 4096: 10.5 against 10.9, 4096 x 14336: 20.5 against 21.2; 4096 x 13696 is the one
+  // shape it loses, 19.8 against 18.5); at 5 its registers double (12288 x 4096: 22.1 against 18.8).
+  if (m == 1) {
     launch<16, 1, kGated, kAct>(x, x_stride, weight, weight_stride, y, y_stride, m, n, k, s, re);
-  else if (m == 2)
+  } else if (m == 2) {
     launch<8, 2, kGated, kAct>(x, x_stride, weight, weight_stride, y, y_stride, m, n, k, s, re);
-  else if (m <= 4)
+  } else if (m <= 4) {
     launch<8, 4, kGated, kAct>(x, x_stride, weight, weight_stride, y, y_stride, m, n, k, s, re);
-  else if constexpr (!kGated) {
-    if (m <= 8)
-      launch<8, 8, false, kAct>(x, x_stride, weight, weight_stride, y, y_stride, m, n, k, s, re);
-    else
-      launch<2, 16, false, kAct>(x, x_stride, weight, weight_stride, y, y_stride, m, n, k, s, re);
+  } else if constexpr (!kGated) {
+    launch_mfma<kAct, kNoRope>(x, x_stride, weight, weight_stride, y, y_stride, m, n, k, s, re);
   }
   return skv_check_launch(what);
 }
@@ -381,7 +575,7 @@ void launch_qkv_rope(const uint16_t* x, int64_t xs, const uint16_t* w, int64_t w
   if (m == 1) launch<16, 1, false, false, kRope>(x, xs, w, ws, nullptr, 0, m, n, k, s, re);
   else if (m == 2) launch<8, 2, false, false, kRope>(x, xs, w, ws, nullptr, 0, m, n, k, s, re);
   else if (m <= 4) launch<8, 4, false, false, kRope>(x, xs, w, ws, nullptr, 0, m, n, k, s, re);
-  else launch<8, 8, false, false, kRope>(x, xs, w, ws, nullptr, 0, m, n, k, s, re);
+  else launch_mfma<false, kRope>(x, xs, w, ws, nullptr, 0, m, n, k, s, re);
 }
 
 }  // namespace

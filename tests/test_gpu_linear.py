@@ -80,6 +80,26 @@ def test_linear_random_shapes(gpu):
         assert_bf16_close(out.cpu(), want.to(torch.bfloat16), floor=1e-3, what=f"linear random case {case}")
 
 
+@pytest.mark.parametrize("rows", [5, 8, 9, 16])
+@pytest.mark.parametrize("n,k", [(1, 8), (8, 128), (15, 120), (17, 136), (2048, 264), (2049, 2048), (4096, 1024),
+                                 (4097, 1032), (8193, 128)])
+def test_linear_matrix_core_edges(gpu, rows, n, k):
+    """The 5..16-row form at its edges: 8- and 16-row x tiles, weight tiles of 8 and 16 rows with and
+    without a remainder, 4 / 8 / 16 waves, K below, at and past one 128-element block; bound: one bf16
+    rounding (2^-8) of sums whose fp32 order differs (k * 2^-24 of the sum of magnitudes)."""
+    _say(f"linear edges rows={rows} n={n} k={k}")
+    g = torch.Generator().manual_seed(rows * 31 + n * 7 + k)
+    x = torch.randn(rows, k + 8, generator=g).to(torch.bfloat16)[:, :k]
+    w = (torch.randn(n, k + 8, generator=g) / k ** 0.5).to(torch.bfloat16)[:, :k]
+    out = torch.full((rows, n + 3), 7.0, dtype=torch.bfloat16, device=gpu)
+    shadowkv.linear(x.to(gpu), w.to(gpu), out[:, :n])
+    torch.cuda.synchronize()
+    want = x.double() @ w.double().t()
+    lim = want.abs() * 2 ** -8 + k * 2 ** -24 * (x.double().abs() @ w.double().abs().t()) + 1e-30
+    assert ((out[:, :n].cpu().double() - want).abs() <= lim).all()
+    assert (out[:, n:] == 7.0).all(), "wrote outside the output rows"
+
+
 def test_linear_strided_views(gpu):
     """Rows taken from wider buffers (x a column slice, out a slice of a fused output), as the
     decode step passes views of its fused projections."""
