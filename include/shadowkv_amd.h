@@ -393,6 +393,19 @@ int skv_select_outliers(const float* min_cos, int rows, int chunks, int outliers
 int skv_gather_rows(const uint16_t* src, int rows, int src_rows, const int64_t* idx, int dst_rows, uint16_t* dst,
                     void* stream);
 
+/* Causal prompt attention (the prefill attention of the sparse layer, models/attention/shadow.py:12-19):
+ * out[b, i, hq, :] = softmax over j <= i of (scale * q[b, hq, i] . k[b, hq / G, j]) . v[b, hq / G, j],
+ * G = q_heads / kv_heads, 128-element bf16 rows with unit element stride, fp32 scores, probabilities
+ * and sums, one rounding to bf16. q, k, v: 16-byte aligned rows (strides multiples of 8 elements; a
+ * stride may be 0), out 8-byte. workspace: skv_prefill_attn_workspace_bytes bytes, 16-byte aligned
+ * (the transposed values), overwritten. */
+int64_t skv_prefill_attn_workspace_bytes(int batch_size, int kv_heads, int len);
+int skv_prefill_attn(const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_s, const uint16_t* k,
+                     int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_s, const uint16_t* v,
+                     int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_s, uint16_t* out, int64_t o_stride_b,
+                     int64_t o_stride_s, int64_t o_stride_h, int batch_size, int q_heads, int kv_heads, int len,
+                     float scale, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* The value fetch of the misses and the key rebuild in one launch: the work of
  * skv_gather_copy_misses_with_offsets(values, v_cache_buffer, offsets, cnts, batch_size, heads,
  * cpu_v_length, num_chunks*chunk_size*head_dim, gpu_v_offset, gpu_v_stride, num_chunks,

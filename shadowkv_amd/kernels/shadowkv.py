@@ -1018,6 +1018,27 @@ def gather_rows(src, idx, dst):
               dst.data_ptr(), _stream())
 
 
+def prefill_attn(q, k, v):
+    """Causal GQA attention of a whole prompt, fp32 scores, probabilities and sums: q [B, Hq, L, 128],
+    k / v [B, Hkv, L, 128] (bf16, any strides) -> [B, L, Hq, 128]. The values are transposed into a
+    workspace of their size first."""
+    B, Hq, L, D = q.shape
+    H = k.shape[1]
+    for t, nm in ((q, "q"), (k, "k"), (v, "v")):
+        _dev(t, nm, torch.bfloat16)
+    if D != 128 or k.shape != (B, H, L, D) or v.shape != k.shape or Hq % H or q.numel() == 0:
+        raise ValueError(f"prefill_attn: q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)}")
+    q, k, v = (t if t.stride(3) == 1 and t.data_ptr() % 16 == 0 and not any(s % 8 for s in t.stride()[:3])
+               else t.clone(memory_format=torch.contiguous_format) for t in (q, k, v))
+    out = torch.empty(B, L, Hq, D, dtype=q.dtype, device=q.device)
+    nbytes = _lib.lib().skv_prefill_attn_workspace_bytes(B, H, L)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+    _lib.call("skv_prefill_attn", q.data_ptr(), *q.stride()[:3], k.data_ptr(), *k.stride()[:3], v.data_ptr(),
+              *v.stride()[:3], out.data_ptr(), *out.stride()[:3], B, Hq, H, L, 1.0 / math.sqrt(D), ws.data_ptr(),
+              nbytes, _stream())
+    return out
+
+
 # ---------------------------------------------------------------------------------------------
 # f3: device chunk pool
 
