@@ -393,6 +393,18 @@ int skv_select_outliers(const float* min_cos, int rows, int chunks, int outliers
 int skv_gather_rows(const uint16_t* src, int rows, int src_rows, const int64_t* idx, int dst_rows, uint16_t* dst,
                     void* stream);
 
+/* The `rank` leading eigenpairs of `batch` symmetric positive semidefinite fp32 matrices a [batch, n, n]
+ * (the keys' Gram matrices of the prompt factorisation, in place of the SVD at models/kvcache/shadow.py:426):
+ * w [batch, rank] eigenvalues, descending; vt [batch, rank, n] their orthonormal eigenvectors, rows;
+ * status [batch] 1 where the problem was solved. A status other than 1 leaves w and vt undefined: a
+ * largest diagonal entry that is zero, not finite or beyond 2^+-100, or workgroups that did not come to run
+ * beside one another in time (every wait is bounded). Eigenvalues closer than about 1e-9 of the largest
+ * may have eigenvectors that are not orthogonal; callers check. batch <= 8 (one problem per XCD),
+ * 2 <= n <= 1024, 1 <= rank <= n. workspace: skv_sym_eig_workspace_bytes bytes, 16-byte aligned. */
+int64_t skv_sym_eig_workspace_bytes(int batch, int n, int rank);
+int skv_sym_eig_top(const float* a, int batch, int n, int rank, float* w, float* vt, int32_t* status, void* workspace,
+                    int64_t workspace_bytes, void* stream);
+
 /* Causal prompt attention (the prefill attention of the sparse layer, models/attention/shadow.py:12-19):
  * out[b, i, hq, :] = softmax over j <= i of (scale * q[b, hq, i] . k[b, hq / G, j]) . v[b, hq / G, j],
  * G = q_heads / kv_heads, 128-element bf16 rows with unit element stride, fp32 scores, probabilities

@@ -1018,6 +1018,28 @@ def gather_rows(src, idx, dst):
               dst.data_ptr(), _stream())
 
 
+SYM_EIG_MAX_N = 1024
+SYM_EIG_MAX_BATCH = 8
+
+
+def sym_eig_top(a, rank):
+    """The `rank` leading eigenpairs of symmetric positive semidefinite a [b, n, n] (fp32, contiguous,
+    b <= 8, 2 <= n <= 1024): (w [b, rank] descending, vt [b, rank, n], status [b] int32). Only rows of
+    status 1 hold a result, whose orthogonality within clusters of eigenvalues is the caller's to check."""
+    _dev(a, "a", torch.float32)
+    if a.dim() != 3 or a.shape[1] != a.shape[2] or not a.is_contiguous():
+        raise ValueError(f"sym_eig_top: a {tuple(a.shape)} must be contiguous [b, n, n]")
+    b, n, _ = a.shape
+    w = torch.empty(b, rank, dtype=torch.float32, device=a.device)
+    vt = torch.empty(b, rank, n, dtype=torch.float32, device=a.device)
+    status = torch.empty(b, dtype=torch.int32, device=a.device)
+    nbytes = max(16, _lib.lib().skv_sym_eig_workspace_bytes(b, n, rank))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=a.device)
+    _lib.call("skv_sym_eig_top", a.data_ptr(), b, n, rank, w.data_ptr(), vt.data_ptr(), status.data_ptr(),
+              ws.data_ptr(), nbytes, _stream())
+    return w, vt, status
+
+
 def prefill_attn(q, k, v):
     """Causal GQA attention of a whole prompt, fp32 scores, probabilities and sums: q [B, Hq, L, 128],
     k / v [B, Hkv, L, 128] (bf16, any strides) -> [B, L, Hq, 128]. The values are transposed into a

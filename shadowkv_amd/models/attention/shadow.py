@@ -10,28 +10,21 @@ where that kernel does not apply).
 import math
 
 import torch
-from torch.autograd import forward_ad
 
 from ...kernels import shadowkv
-from ..tensor_op import repeat_kv
+from ..tensor_op import plain_eager, repeat_kv
 from .base import AttentionBase
 
 
 def _kernel_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
-    """Whether the prompt attention kernel serves this call: plain bf16 device tensors of 128-dim heads
-    and one length, not differentiated (backward, forward mode or a functorch transform) and not traced
-    (compile, a dispatch mode), where the torch operations have to be seen."""
-    ts = (q, k, v)
-    if not all(type(t) is torch.Tensor and t.is_cuda and t.dtype == torch.bfloat16 and t.dim() == 4 for t in ts):
+    """Whether the prompt attention kernel serves this call: bf16 tensors of 128-dim heads and one
+    length, outside autograd and tracing."""
+    if not (plain_eager(q, k, v) and all(t.dtype == torch.bfloat16 and t.dim() == 4 for t in (q, k, v))):
         return False
     B, Hq, L, D = q.shape
     H = k.shape[1]
     return (D == 128 and k.shape == (B, H, L, D) and v.shape == k.shape and q.numel() > 0 and H > 0 and Hq % H == 0
-            and B * Hq * L < 2 ** 31 and B * H <= 65535 and q.device == k.device == v.device
-            and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
-            and forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
-            and torch._C._len_torch_dispatch_stack() == 0 and not torch.compiler.is_compiling()
-            and not torch.jit.is_tracing())
+            and B * Hq * L < 2 ** 31 and B * H <= 65535)
 
 
 def causal_attention_fp32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, block: int = 1024) -> torch.Tensor:

@@ -9,8 +9,20 @@ in models/llama.py:138-142 ([cos(64) | sin(64)] rows) and models/glm.py:132-133
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 
 from ..kernels import shadowkv
+
+
+def plain_eager(*tensors: torch.Tensor) -> bool:
+    """Whether a call on these tensors may leave torch's operators for a kernel: plain device tensors on
+    one device, not differentiated (backward, forward mode or a functorch transform) and not traced
+    (compile, jit, a dispatch mode), where the torch operations have to be seen."""
+    return (all(type(t) is torch.Tensor and t.is_cuda and t.device == tensors[0].device for t in tensors)
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+            and forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0 and not torch.compiler.is_compiling()
+            and not torch.jit.is_tracing())
 
 
 def repeat_kv(hidden_states: torch.Tensor, n_rep: int) -> torch.Tensor:

@@ -1,0 +1,93 @@
+"""The leading eigenpairs of symmetric positive semidefinite matrices (skv_sym_eig_top) against the
+float64 eigendecomposition, and the factors where the kernel's result is not taken."""
+import pytest
+import torch
+
+from shadowkv_amd.kernels import shadowkv
+from shadowkv_amd.models.kvcache import shadow as kv
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(msg):
+    print(msg, flush=True)
+
+
+def _check(a, rank, scale=1.0):
+    """Residuals, orthogonality and eigenvalues within n * 2^-24 of the largest eigenvalue (the backward
+    error of a Householder reduction in fp32)."""
+    w, vt, status = shadowkv.sym_eig_top(a, rank)
+    torch.cuda.synchronize()
+    assert (status.cpu() == 1).all()
+    b, n, _ = a.shape
+    lim = max(n, 64) * 2 ** -24
+    A, W, V = a.cpu().double(), w.cpu().double(), vt.cpu().double()
+    want = torch.linalg.eigvalsh(A).flip(-1)[:, :rank]
+    top = want[:, :1]
+    assert ((W - want).abs() <= lim * top).all()
+    assert ((V @ A - W.unsqueeze(-1) * V).norm(dim=-1) <= lim * top).all()
+    assert ((V @ V.transpose(1, 2) - torch.eye(rank, dtype=torch.float64)).abs() <= lim).all()
+
+
+# Sizes at, below and past the register tiles (64 NR rows: 128, 256, 512, 1024) and phases.
+@pytest.mark.parametrize("b,n,rank", [(1, 2, 2), (1, 3, 1), (8, 17, 17), (1, 64, 16), (2, 127, 40), (1, 128, 128), (1, 129, 7),
+                                      (3, 256, 160), (1, 300, 12), (1, 512, 160), (2, 513, 20), (1, 1000, 160),
+                                      (1, 1023, 3), (2, 1024, 160)])
+def test_sym_eig_top(gpu, b, n, rank):
+    _say(f"sym_eig_top b={b} n={n} rank={rank}")
+    g = torch.Generator().manual_seed(n + rank)
+    x = torch.randn(b, 2 * n + 5, n, generator=g) * torch.logspace(0.5, -0.5, n)
+    a = (x.transpose(1, 2) @ x * 2.0 ** (n % 40 - 20)).to(gpu)
+    a = (0.5 * (a + a.transpose(1, 2))).contiguous()
+    _check(a, rank)
+
+
+@pytest.mark.parametrize("kind", ["low rank", "diagonal", "steep", "one entry"])
+def test_sym_eig_top_special_spectra(gpu, kind):
+    """Reflections of zero columns, split tridiagonals and eigenvalues down to rounding noise."""
+    _say(f"sym_eig_top {kind}")
+    g = torch.Generator().manual_seed(5)
+    n = 256
+    if kind == "low rank":
+        x = torch.randn(1, 600, 40, generator=g) @ torch.randn(1, 40, n, generator=g)
+        rank = 40
+    elif kind == "diagonal":
+        x, rank = torch.diag(torch.linspace(1, 3, n))[None], 30
+    elif kind == "steep":
+        x, rank = torch.randn(1, 600, n, generator=g) * torch.logspace(0, -6, n), 30
+    else:
+        x, rank = torch.zeros(1, n, n), 1
+        x[0, 70, 70] = 2.0
+    _check((x.transpose(1, 2) @ x).contiguous().to(gpu), rank)
+
+
+def test_factors_fall_back(gpu):
+    """A zero or non-finite matrix is refused by its status, an exactly degenerate one by the
+    orthogonality check; low_rank_factors then gives what eigh gives, and what eigh refuses stays refused."""
+    _say("eigen fallback")
+    n = 128
+    for a in (torch.zeros(1, n, n), torch.full((1, n, n), float("nan"))):
+        _, _, status = shadowkv.sym_eig_top(a.to(gpu), 8)
+        assert status.cpu().tolist() == [0]
+    eye = torch.eye(n, device=gpu)[None].contiguous()
+    assert kv._top_eigenpairs(eye, 8) is None
+    assert kv._top_eigenpairs(eye[:, :32, :32].contiguous(), 8) is None  # small: eigh
+    u, svt = kv.low_rank_factors(torch.eye(n, device=gpu)[None].to(torch.bfloat16), 8)
+    assert (svt @ svt.transpose(1, 2) - torch.eye(8, device=gpu)).abs().max() < 1e-5
+    assert torch.isfinite(u).all()
+    k = torch.randn(1, 300, n, device=gpu, requires_grad=True)
+    u, svt = kv.low_rank_factors(k, 8)
+    (u @ svt).sum().backward()
+    assert torch.isfinite(k.grad).all()
+
+
+def test_batches_past_the_xcds(gpu):
+    """More problems than one call takes (8) are split."""
+    _say("eigen batch 9")
+    g = torch.Generator().manual_seed(1)
+    k = torch.randn(9, 200, 96, generator=g).to(gpu)
+    u, svt = kv.low_rank_factors(k, 20)
+    uu, s, vh = torch.linalg.svd(k.cpu().double(), full_matrices=False)
+    want = (uu[..., :20] * s[:, None, :20]) @ vh[:, :20]
+    got = (u @ svt).cpu().double()
+    assert ((got - want).norm(dim=(1, 2)) / want.norm(dim=(1, 2))).max() < 1e-3
