@@ -21,8 +21,9 @@
 // all), the polling loads agent-scope (past the L1). Every wait is bounded: a workgroup that waits too long
 // gives up for good, the problem's status says so and the caller takes another way.
 //
-// MI355X, rank 160, us: n = 1024: 1700 + 460 + 227 (reduction + eigenpairs of T + back transformation; 1.7
-// a step), n = 512: 620 + 232 + 93, n = 256: 270 + 118 + 39; rocSOLVER's full decomposition 19600, 10400, 4900.
+// MI355X, rank 160, us in all: n = 1024 2290 (the reduction 1640, 1.6 a step; the eigenpairs of T 460; the
+// back transformation 180), n = 512 909, n = 256 416 (1.0 a step: the exchange and the chain of
+// reductions alone); rocSOLVER's full decomposition 19600, 10400, 4900.
 #include <type_traits>
 
 #include "wave_reduce.h"
@@ -115,10 +116,17 @@ struct Reduction {
       // Reflection of column i: v = (0 .., 1, x), H = I - tau v v^T maps the column to (.., beta, 0 ..).
       const float di = pick<R0, R1>(a, i), alpha = pick<R0, R1>(a, i + 1);
       float beta = alpha, tau = 0.f, inv = 0.f;
-      if (nn > 0.f) {
-        beta = -copysignf(sqrtf(fmaf(alpha, alpha, nn)), alpha);
-        tau = (beta - alpha) / beta;
-        inv = 1.f / (alpha - beta);
+      if (nn > 1e-36f) {
+        // 1 / |beta| and 1 / (alpha - beta) from the hardware estimates and a Newton step each: the
+        // divisions and the square root would lie on every step's critical path.
+        const float sq = fmaf(alpha, alpha, nn);
+        float rs = __builtin_amdgcn_rsqf(sq);
+        rs = fmaf(0.5f * rs, fmaf(-sq * rs, rs, 1.f), rs);
+        beta = -copysignf(sq * rs, alpha);
+        tau = fmaf(fabsf(alpha), rs, 1.f);  // (beta - alpha) / beta
+        const float den = alpha - beta;
+        inv = __builtin_amdgcn_rcpf(den);
+        inv = fmaf(fmaf(-den, inv, 1.f), inv, inv);
       }
       Col v;
 #pragma unroll
@@ -240,13 +248,14 @@ struct Reduction {
 // (One wave per SIMD with up to 512 registers: 8 columns of 1024 rows are 128 of them; two waves of
 // 4 columns would do the redundant vector work twice.)
 // A workgroup takes its part by its order of arrival on its XCD: problem b runs on XCD b, its
-// 2 NR workgroups one per CU (see pc).
+// 2 NR workgroups one per CU on an idle device (a
+// request for LDS that forces it changes nothing, and small workgroups let two calls run side by side).
 template <int NR>
 __global__ void __launch_bounds__(kWgWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 tridiag_kernel(EigenArgs g) {
   using Red = Reduction<NR>;
   // Two of the buffers are used; the size keeps a second workgroup off the CU (160 KB of LDS).
-  __shared__ float2 pc[88 * 1024 / (8 * Red::kPad)][Red::kPad];
+  __shared__ float2 pc[2][Red::kPad];
   __shared__ int part;
   const int b = static_cast<int>(__builtin_amdgcn_s_getreg(kHwRegXccId) & 15u);
   if (b >= g.batch) return;
@@ -333,7 +342,8 @@ __global__ void __launch_bounds__(64) bisect_kernel(EigenArgs g, int npad) {
   hi += 1e-12 * norm;
   // 64 interior points split [lo, hi] into 65 parts; lambda_k >= x when at least k + 1 eigenvalues are
   // not below x, and the eigenvalues below x are the sign changes of the minors p_i (an exact zero
-  // between two nonzero minors counts once with either sign). 9 passes: 65^-9 of the width.
+  // between two nonzero minors counts once with either sign). 9 passes: 65^-9 of the
+  // width (8, 3e-15, are not enough for the vectors of a spectrum that ends in rounding noise).
   for (int pass = 0; pass < 9; ++pass) {
     const double step = (hi - lo) / 65.0;
     const double x = lo + step * (lane + 1);
@@ -432,22 +442,30 @@ __global__ void __launch_bounds__(64) bisect_kernel(EigenArgs g, int npad) {
   if (lane == 0) g.w[b * g.rank + k] = static_cast<float>(lam * static_cast<double>(g.scale[b]));
 }
 
-// vt[k] = H_0 H_1 ... H_{n-2} z_k, one wave per vector, the reflections requested kAhead steps ahead.
+// vt[k] = H_0 H_1 ... H_{n-2} z_k, one wave per vector, the reflections requested kAhead steps ahead in
+// 16-byte loads (the loads bound it: 4-byte ones took 227 against 180 us at n = 1024; two reflections
+// per round of reductions were no faster).
 template <int NR>
 __global__ void __launch_bounds__(64) backtransform_kernel(EigenArgs g) {
-  constexpr int kPad = 64 * NR, kAhead = 4;
+  constexpr int kPad = 64 * NR, kAhead = 8;
   const int b = blockIdx.y, k = blockIdx.x, n = g.n, lane = threadIdx.x;
   if (g.status[b] != 1) return;
   const float* vb = g.v + static_cast<int64_t>(b) * n * kPad;
   const float* tau = g.tau + b * kPad;
-  float z[NR];
+  // Register r holds row row0(r) = 64 VL (r / VL) + VL lane + r % VL: VL rows, one load, side by side.
+  constexpr int VL = NR >= 4 ? 4 : 2;
+  typedef float Vec __attribute__((ext_vector_type(VL)));
+  Vec z[NR / VL];
+  const float* zs = g.z + (static_cast<int64_t>(b) * g.rank + k) * kPad + VL * lane;
 #pragma unroll
-  for (int r = 0; r < NR; ++r) z[r] = g.z[(static_cast<int64_t>(b) * g.rank + k) * kPad + 64 * r + lane];
-  float v[kAhead][NR], t[kAhead];
-  auto load = [&](int i, float* dst, float& tt) {
+  for (int r = 0; r < NR / VL; ++r) z[r] = *reinterpret_cast<const Vec*>(zs + 64 * VL * r);
+  Vec v[kAhead][NR / VL];
+  float t[kAhead];
+  auto load = [&](int i, Vec* dst, float& tt) {
     const int ii = max(i, 0);
 #pragma unroll
-    for (int r = 0; r < NR; ++r) dst[r] = vb[static_cast<int64_t>(ii) * kPad + 64 * r + lane];
+    for (int r = 0; r < NR / VL; ++r)
+      dst[r] = *reinterpret_cast<const Vec*>(vb + static_cast<int64_t>(ii) * kPad + VL * lane + 64 * VL * r);
     tt = i < 0 ? 0.f : tau[ii];
   };
 #pragma unroll
@@ -457,17 +475,19 @@ __global__ void __launch_bounds__(64) backtransform_kernel(EigenArgs g) {
     for (int u = 0; u < kAhead; ++u) {
       float s = 0.f;
 #pragma unroll
-      for (int r = 0; r < NR; ++r) s = fmaf(v[u][r], z[r], s);
+      for (int r = 0; r < NR; ++r) s = fmaf(v[u][r / VL][r % VL], z[r / VL][r % VL], s);
       s = skv::wave_sum_dpp(s) * t[u];
 #pragma unroll
-      for (int r = 0; r < NR; ++r) z[r] = fmaf(-s, v[u][r], z[r]);
+      for (int r = 0; r < NR; ++r) z[r / VL][r % VL] = fmaf(-s, v[u][r / VL][r % VL], z[r / VL][r % VL]);
       load(i - u - kAhead, v[u], t[u]);
     }
   }
   float* out = g.vt + (static_cast<int64_t>(b) * g.rank + k) * n;
 #pragma unroll
-  for (int r = 0; r < NR; ++r)
-    if (64 * r + lane < n) out[64 * r + lane] = z[r];
+  for (int r = 0; r < NR; ++r) {
+    const int row = 64 * VL * (r / VL) + VL * lane + r % VL;
+    if (row < n) out[row] = z[r / VL][r % VL];
+  }
 }
 
 __global__ void __launch_bounds__(256) prepare_kernel(ulonglong2* xchg, int64_t count, uint32_t* tickets,
