@@ -405,6 +405,25 @@ int64_t skv_sym_eig_workspace_bytes(int batch, int n, int rank);
 int skv_sym_eig_top(const float* a, int batch, int n, int rank, float* w, float* vt, int32_t* status, void* workspace,
                     int64_t workspace_bytes, void* stream);
 
+/* Gram matrices of a prompt's pre-RoPE keys, read in place: keys (b, row, head, 128 dims) bf16 at
+ * keys + b*stride_b + row*stride_s + head*stride_h (elements, multiples of 8; 16-byte aligned) ->
+ * gram [batch, n, n] fp32, n = heads * 128 <= 1024, column head*128 + d: exact bf16 products, fp32 sums over
+ * shares of the rows, added in fp64. workspace: skv_keys_gram_workspace_bytes bytes, 16-byte aligned. */
+int64_t skv_keys_gram_workspace_bytes(int batch, int rows, int heads);
+int skv_keys_gram(const uint16_t* keys, int64_t stride_b, int64_t stride_h, int64_t stride_s, int batch, int rows,
+                  int heads, float* gram, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* The rank-R factors of such keys from the Gram matrix's leading eigenpairs (w [batch, rank], vt [batch,
+ * rank, n] rows): u[b, row, r] = bf16(sum_c keys[row, c] vt[r, c] / s_r), s = sqrt(max(w, 0)) (rows of rank
+ * elements, batch stride u_stride_b), and sv[b, head, d, r] = bf16(s_r vt[r, head*128 + d]) (batch stride
+ * sv_stride_b) - get_svd, models/kvcache/shadow.py:411-444. Products with the fp32 vt are exact (three
+ * bf16 parts), sums fp32. rank: a multiple of 4 up to n; u 8-byte aligned. workspace:
+ * skv_keys_factors_workspace_bytes bytes, 16-byte aligned. */
+int64_t skv_keys_factors_workspace_bytes(int batch, int heads, int rank);
+int skv_keys_factors(const uint16_t* keys, int64_t stride_b, int64_t stride_h, int64_t stride_s, int batch, int rows,
+                     int heads, const float* w, const float* vt, int rank, uint16_t* u, int64_t u_stride_b,
+                     uint16_t* sv, int64_t sv_stride_b, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Causal prompt attention (the prefill attention of the sparse layer, models/attention/shadow.py:12-19):
  * out[b, i, hq, :] = softmax over j <= i of (scale * q[b, hq, i] . k[b, hq / G, j]) . v[b, hq / G, j],
  * G = q_heads / kv_heads, 128-element bf16 rows with unit element stride, fp32 scores, probabilities

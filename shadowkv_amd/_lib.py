@@ -74,6 +74,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "skv_chunk_stats": (_i32, [_p, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _p, _p, _p]),
     "skv_select_outliers": (_i32, [_p, _i32, _i32, _i32, _p, _p, _p]),
     "skv_gather_rows": (_i32, [_p, _i32, _i32, _p, _i32, _p, _p]),
+    "skv_keys_gram_workspace_bytes": (_i64, [_i32, _i32, _i32]),
+    "skv_keys_gram": (_i32, [_p, _i64, _i64, _i64, _i32, _i32, _i32, _p, _p, _i64, _p]),
+    "skv_keys_factors_workspace_bytes": (_i64, [_i32, _i32, _i32]),
+    "skv_keys_factors": (_i32, [_p, _i64, _i64, _i64, _i32, _i32, _i32, _p, _p, _i32, _p, _i64, _p, _i64, _p, _i64,
+                                _p]),
     "skv_sym_eig_workspace_bytes": (_i64, [_i32, _i32, _i32]),
     "skv_sym_eig_top": (_i32, [_p, _i32, _i32, _i32, _p, _p, _p, _p, _i64, _p]),
     "skv_prefill_attn_workspace_bytes": (_i64, [_i32, _i32, _i32]),

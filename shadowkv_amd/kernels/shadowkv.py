@@ -1018,6 +1018,50 @@ def gather_rows(src, idx, dst):
               dst.data_ptr(), _stream())
 
 
+KEYS_MAX_COLUMNS = 1024
+
+
+def _keys4(keys: torch.Tensor):
+    _dev(keys, "keys", torch.bfloat16)
+    if keys.dim() != 4 or keys.shape[-1] != 128 or keys.stride(-1) != 1:
+        raise ValueError(f"keys {tuple(keys.shape)} must be [b, rows, heads, 128] with contiguous heads")
+    b, rows, heads, _ = keys.shape
+    return b, rows, heads, (keys.stride(0), keys.stride(2), keys.stride(1))
+
+
+def keys_gram(keys):
+    """Gram matrices [b, n, n] (fp32) of a prompt's pre-RoPE keys [b, rows, heads, 128] (bf16, any (b, row,
+    head) strides of multiples of 8, 16-byte aligned), n = heads * 128 <= 1024."""
+    b, rows, heads, strides = _keys4(keys)
+    n = heads * 128
+    gram = torch.empty(b, n, n, dtype=torch.float32, device=keys.device)
+    nbytes = max(16, _lib.lib().skv_keys_gram_workspace_bytes(b, rows, heads))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=keys.device)
+    _lib.call("skv_keys_gram", keys.data_ptr(), *strides, b, rows, heads, gram.data_ptr(), ws.data_ptr(), nbytes,
+              _stream())
+    return gram
+
+
+def keys_factors(keys, w, vt, u, sv):
+    """Rank-R factors of keys [b, rows, heads, 128] from its Gram matrix's leading eigenpairs (w [b, R], vt
+    [b, R, n]) into u [b, rows, R] and sv [b, heads, 128, R] (bf16, contiguous per sequence): u = keys V / s
+    and sv = diag(s) V^T per head, s = sqrt(w)."""
+    b, rows, heads, strides = _keys4(keys)
+    rank = w.shape[-1]
+    _dev(w, "w", torch.float32), _dev(vt, "vt", torch.float32)
+    _dev(u, "u", torch.bfloat16), _dev(sv, "sv", torch.bfloat16)
+    if w.shape != (b, rank) or vt.shape != (b, rank, heads * 128) or u.shape != (b, rows, rank) or \
+            sv.shape != (b, heads, 128, rank):
+        raise ValueError(f"keys_factors: keys {tuple(keys.shape)} w {tuple(w.shape)} vt {tuple(vt.shape)} "
+                         f"u {tuple(u.shape)} sv {tuple(sv.shape)}")
+    if not (w.is_contiguous() and vt.is_contiguous() and u[0].is_contiguous() and sv[0].is_contiguous()):
+        raise ValueError("keys_factors: w, vt and each sequence's u and sv must be contiguous")
+    nbytes = max(16, _lib.lib().skv_keys_factors_workspace_bytes(b, heads, rank))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=keys.device)
+    _lib.call("skv_keys_factors", keys.data_ptr(), *strides, b, rows, heads, w.data_ptr(), vt.data_ptr(), rank,
+              u.data_ptr(), u.stride(0), sv.data_ptr(), sv.stride(0), ws.data_ptr(), nbytes, _stream())
+
+
 SYM_EIG_MAX_N = 1024
 SYM_EIG_MAX_BATCH = 8
 

@@ -1,0 +1,99 @@
+"""The Gram matrix and the factors of a prompt's keys read in place (skv_keys_gram, skv_keys_factors)
+against float64, and get_svd by either route."""
+import types
+
+import pytest
+import torch
+
+from shadowkv_amd.kernels import shadowkv
+from shadowkv_amd.models.kvcache import ShadowKVCache_CPU
+from shadowkv_amd.models.kvcache import shadow as kv
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(msg):
+    print(msg, flush=True)
+
+
+# Rows around one stage (64), one share and the 256-row blocks; one to eight heads (half, whole and several
+# 256-column tiles); ranks of one, a partial and five vector tiles; by head, by token, and padded rows.
+@pytest.mark.parametrize("b,rows,H,R,layout", [(1, 1, 1, 4, "token"), (2, 63, 1, 32, "head"), (1, 65, 2, 48, "padded"),
+                                               (3, 257, 3, 160, "head"), (1, 511, 8, 36, "token"),
+                                               (1, 1025, 4, 320, "padded"), (1, 33000, 1, 128, "head"),
+                                               (1, 33001, 2, 160, "token")])
+def test_gram_and_factors(gpu, b, rows, H, R, layout):
+    """Bounds: a Gram entry is one fp32 sum of exact products (rows * 2^-24 of the sum of magnitudes, ample);
+    a factor one fp32 sum of n products, one division and one rounding to bf16."""
+    _say(f"gram and factors b={b} rows={rows} H={H} R={R} {layout}")
+    g = torch.Generator().manual_seed(rows + H)
+    n = H * 128
+    k = torch.randn(b, rows, H, 128, generator=g).to(torch.bfloat16)
+    if layout == "head":
+        dev = k.transpose(1, 2).contiguous().to(gpu).transpose(1, 2)
+    elif layout == "padded":
+        dev = torch.full((b, rows + 2, H, 136), float("nan"), dtype=torch.bfloat16, device=gpu)[:, 1:-1, :, :128]
+        dev.copy_(k)
+    else:
+        dev = k.to(gpu)
+    K = k.view(b, rows, n).double()
+    gram = shadowkv.keys_gram(dev)
+    want = K.transpose(1, 2) @ K
+    assert ((gram.cpu().double() - want).abs() <= rows * 2 ** -24 * (K.abs().transpose(1, 2) @ K.abs()) + 1e-30).all()
+    assert torch.equal(gram, gram.transpose(1, 2))
+
+    V = torch.linalg.qr(torch.randn(b, n, max(R, 1), generator=g))[0][..., :R] if R <= n else torch.randn(b, n, R, generator=g)
+    if R > n:
+        with pytest.raises(RuntimeError):
+            shadowkv.keys_factors(dev, torch.ones(b, R, device=gpu), V.transpose(1, 2).contiguous().to(gpu),
+                                  torch.empty(b, rows, R, dtype=torch.bfloat16, device=gpu),
+                                  torch.empty(b, H, 128, R, dtype=torch.bfloat16, device=gpu))
+        return
+    w = torch.rand(b, R, generator=g) * 4 + 0.5
+    vt = V.transpose(1, 2).contiguous()
+    u = torch.full((b, rows, R), 7.0, dtype=torch.bfloat16, device=gpu)
+    sv = torch.full((b, H, 128, R), 7.0, dtype=torch.bfloat16, device=gpu)
+    shadowkv.keys_factors(dev, w.to(gpu), vt.to(gpu), u, sv)
+    s = w.double().sqrt()
+    U = (K @ vt.double().transpose(1, 2)) / s.unsqueeze(1)
+    lim = U.abs() * (2 ** -8 + 2 ** -20) + n * 2 ** -24 * (K.abs() @ vt.double().abs().transpose(1, 2)) / s.unsqueeze(1)
+    assert ((u.cpu().double() - U).abs() <= lim + 1e-30).all()
+    S = (s.unsqueeze(-1) * vt.double()).view(b, R, H, 128).permute(0, 2, 3, 1)
+    assert ((sv.cpu().double() - S).abs() <= S.abs() * (2 ** -8 + 2 ** -20)).all()
+
+
+@pytest.mark.parametrize("form", ["head", "token", "odd"])
+def test_get_svd_routes(gpu, form, monkeypatch):
+    """get_svd through the kernels and through the torch operations: the same reconstruction, for keys by
+    head, fused by token, and at an odd offset (which only the torch operations take)."""
+    _say(f"get_svd {form}")
+    B, H, ctx, R = 2, 2, 700, 64
+    g = torch.Generator().manual_seed(3)
+    k = (torch.randn(B, ctx, 48, generator=g) @ torch.randn(B, 48, H * 128, generator=g) / 7
+         + 0.05 * torch.randn(B, ctx, H * 128, generator=g)).to(torch.bfloat16).to(gpu)
+    if form == "head":
+        arg = k.view(B, ctx, H, 128).transpose(1, 2).contiguous()
+    elif form == "token":
+        arg = k
+    else:
+        arg = torch.empty(B * ctx * H * 128 + 1, dtype=torch.bfloat16, device=gpu)[1:].view(B, ctx, H * 128)
+        arg.copy_(k)
+    cfg = types.SimpleNamespace(num_attention_heads=2 * H, num_key_value_heads=H, hidden_size=2 * H * 128,
+                                num_hidden_layers=1)
+    rec = []
+    for force in (False, True):
+        cache = ShadowKVCache_CPU(cfg, batch_size=B, max_length=ctx, device=str(gpu), sparse_budget=256, rank=R,
+                                  value_store="device")
+        taken = []
+        real = ShadowKVCache_CPU._keys_in_place
+        monkeypatch.setattr(ShadowKVCache_CPU, "_keys_in_place",
+                            lambda self, x: None if force else (taken.append(real(self, x)) or taken[-1]))
+        cache.get_svd(arg, 0)
+        monkeypatch.setattr(ShadowKVCache_CPU, "_keys_in_place", real)
+        if not force:
+            assert (taken[0] is None) == (form == "odd")
+        rec.append(torch.einsum("bcr,bhdr->bchd", cache.U[0].float(), cache.SV[0].float()).double())
+    diff = (rec[0] - rec[1]).norm() / rec[1].norm()
+    assert diff < 4e-3, diff  # two bf16 roundings of the same fp32 factors, up to their signs
+    err = (rec[0].reshape(B, ctx, -1) - k.double()).norm() / k.double().norm()
+    assert err < 0.08  # the noise outside rank 64
