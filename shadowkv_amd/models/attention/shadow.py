@@ -50,6 +50,14 @@ def causal_attention_fp32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, blo
     return out
 
 
+# Fetch workgroups of a decode() call: with nothing beside the launch but the rebuild, which the host reads
+# slow, more of them in flight win over the default of 64, which suits lanes whose fetches run
+# beside dense layers (MI355X, us per call at 64 / 96 / 128 / 256: 4 x 122880 tokens, 2048 selected, 258 / 246 /
+# 242 / 243; 3 x 28426, 4096 selected, 292 / 259 / 250 / 256; 4 x 50000, 1024 selected in chunks of 4, 157 / 154 /
+# 152 / 154).
+JOINED_FETCH_WORKGROUPS = 128
+
+
 class ShadowAttention(AttentionBase):
 
     def prefill(self, query_states, key_states, value_states, position_ids, layer_idx):
@@ -60,7 +68,22 @@ class ShadowAttention(AttentionBase):
         return causal_attention_fp32(query_states, key_states, value_states)
 
     def decode(self, query_states, key_states, value_states, position_ids, layer_idx):
-        return self.decode_end(self.decode_begin(query_states, key_states, value_states, position_ids, layer_idx))
+        """One new token through the layer: decode_begin() and decode_end(). Nothing can overlap the
+        value fetch from outside here, so a cache in its default setting takes the shortest chain on the
+        current stream: the selection's launch moves both buffers' hits and one launch fetches the missed
+        values beside their keys' rebuild, in place of two compaction launches, two stream hops
+        and two launches side by side (the same buffer contents). MI355X, values in host memory,
+        one sequence of 8192 tokens: 236 -> 144 us, 4 of 122880: 287 -> 242 us."""
+        kv_cache = self.kv_cache
+        if kv_cache.pooled or kv_cache.fold_hit_moves or getattr(kv_cache, "key_stream", None) is not None:
+            return self.decode_end(self.decode_begin(query_states, key_states, value_states, position_ids, layer_idx))
+        query_states, key_states = self.apply_rotary_pos_emb(query_states, key_states, position_ids)
+        kv_cache.update_kv_cache(key_states, value_states, layer_idx)
+        position_ids = kv_cache.get_retrieval_position_ids(layer_idx=layer_idx, query_states=query_states, fold_all=True)
+        key_states, value_states = kv_cache.fetch_and_rebuild(
+            layer_idx, position_ids, self.cos_sin_cache,
+            fetch_workgroups=kv_cache.fused_fetch_workgroups or JOINED_FETCH_WORKGROUPS)
+        return self.decode_end((query_states, key_states, value_states, [], layer_idx))
 
     def decode_begin(self, query_states, key_states, value_states, position_ids, layer_idx):
         """First half of decode(): RoPE, append, chunk selection, the value fetch launched on the

@@ -454,8 +454,11 @@ class ShadowKVCache_CPU(KVCacheBase):
             self.kv_offset = ctx
 
     # ------------------------------------------------------------------ decoding
-    def get_retrieval_position_ids(self, layer_idx: int, query_states: torch.Tensor) -> torch.Tensor:
-        """Select S chunks for the current query and reorder them against the previous slots."""
+    def get_retrieval_position_ids(self, layer_idx: int, query_states: torch.Tensor,
+                                   fold_all: bool = False) -> torch.Tensor:
+        """Select S chunks for the current query and reorder them against the previous slots. fold_all:
+        move both buffers' hits in the same launch, as with fold_hit_moves and one_stream_fetch set, for
+        a fetch_and_rebuild() that follows."""
         B, H, G, D = self.batch_size, self.num_key_value_heads, self.num_key_value_groups, self.head_dim
         self.incoming_q_len = query_states.shape[-2]
         if self.incoming_q_len != 1:
@@ -482,13 +485,14 @@ class ShadowKVCache_CPU(KVCacheBase):
         # chunk_attn; the selected ids in top-k order (selected_chunks) only when keep_selected is set. With
         # fold_hit_moves the same launch also moves the value buffer's hits to their new slots.
         move = None
-        if self.fold_hit_moves and self.values_in_place:
+        both = fold_all or self.one_stream_active()
+        if (fold_all or self.fold_hit_moves) and self.values_in_place:
             # (no value buffer to update: the key buffer's hits, where the key rebuild follows at once)
-            if self.one_stream_active():
+            if both:
                 move = (self.k_cache_buffer[layer_idx], None, self.kernel_offset, self.kernel_stride,
                         self.chunk_size * D)
-        elif self.fold_hit_moves:
-            move = (self.v_cache_buffer[layer_idx], self.k_cache_buffer[layer_idx] if self.one_stream_active() else None,
+        elif fold_all or self.fold_hit_moves:
+            move = (self.v_cache_buffer[layer_idx], self.k_cache_buffer[layer_idx] if both else None,
                     self.kernel_offset, self.kernel_stride, self.chunk_size * D)
         shadowkv.select_chunks(self.gemm_o, self.norm, self.sum, B * H, G, n, self.k_landmark_idx[layer_idx].view(B * H, n),
                                self.select_sets, self.chunks, self.position_ids[layer_idx].view(B * H, -1), self.offsets,
@@ -587,19 +591,23 @@ class ShadowKVCache_CPU(KVCacheBase):
         hits stay in their slots)."""
         return self.one_stream_fetch and (self.pooled or self.fold_hit_moves)
 
-    def fetch_and_rebuild(self, layer_idx: int, position_ids: torch.Tensor, cos_sin_cache: torch.Tensor):
+    def fetch_and_rebuild(self, layer_idx: int, position_ids: torch.Tensor, cos_sin_cache: torch.Tensor,
+                          fetch_workgroups: int | None = None):
         """get_value_cache and get_key_cache as one launch on the current stream: the misses'
         value chunks gathered from the host store beside the misses' key rebuild + RoPE, after a
         selection that moved both buffers' hits (one_stream_fetch). Returns (keys, values), the
         live views of the two buffers. With a chunk pool: the miss list of pool_assign, each miss
-        fetched and rebuilt into its slot of both buffers."""
+        fetched and rebuilt into its slot of both buffers. fetch_workgroups: the fetch workgroups (None:
+        fused_fetch_workgroups)."""
+        if fetch_workgroups is None:
+            fetch_workgroups = self.fused_fetch_workgroups
         if self.pooled:
             B, H, S, D = self.batch_size, self.num_key_value_heads, self.select_sets, self.head_dim
             shadowkv.fetch_misses_rebuild_k_rope_slots(
                 self.v_cache_cpu[layer_idx], self.v_cache_buffer[layer_idx], self.miss_ids.view(B, H, S), self.cnts,
                 self.miss_slot.view(B, H, S), int(self.max_ctx_chunks_len * D), self.sparse_start * D,
                 self.buf_len * D, self.U[layer_idx], self.SV[layer_idx], cos_sin_cache, self.k_cache_buffer[layer_idx],
-                self.sparse_start, self.chunk_size, self.pool_slots, fetch_workgroups=self.fused_fetch_workgroups,
+                self.sparse_start, self.chunk_size, self.pool_slots, fetch_workgroups=fetch_workgroups,
                 rebuild_workgroups=self.fused_rebuild_workgroups)
             return (self._live_view(self.k_cache_buffer[layer_idx], layer_idx),
                     self._live_view(self.v_cache_buffer[layer_idx], layer_idx))
@@ -620,7 +628,7 @@ class ShadowKVCache_CPU(KVCacheBase):
                                              self.kernel_offset, self.kernel_stride, self.U[layer_idx],
                                              self.SV[layer_idx], position_ids, cos_sin_cache,
                                              self.k_cache_buffer[layer_idx], self.sparse_start, self.chunk_size,
-                                             fetch_workgroups=self.fused_fetch_workgroups,
+                                             fetch_workgroups=fetch_workgroups,
                                              rebuild_workgroups=self.fused_rebuild_workgroups)
         return (self._live_view(self.k_cache_buffer[layer_idx], layer_idx),
                 self._live_view(self.v_cache_buffer[layer_idx], layer_idx))

@@ -1,0 +1,68 @@
+"""ShadowAttention.decode (selection with folded hit moves, one fetch + rebuild launch) against
+decode_begin + decode_end (two streams): the same bits in the output, the selection and both buffers."""
+import types
+
+import pytest
+import torch
+
+from shadowkv_amd.decode_model import synthesize_state
+from shadowkv_amd.models.attention import ShadowAttention
+from shadowkv_amd.models.kvcache import ShadowKVCache_CPU
+from shadowkv_amd.models.tensor_op import apply_rotary_pos_emb_cuda, build_cos_sin_cache, build_glm_cos_sin_cache
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(msg):
+    print(msg, flush=True)
+
+
+# One chunk size below, at and above the default, both stores, a selection of the largest size
+# (2048 chunks), both rotary layouts, fetches of fewer and of more tiles than workgroups.
+@pytest.mark.parametrize("B,H,G,ctx,budget,chunk,store,glm", [
+    (1, 8, 4, 6000, 1024, 8, "host", False), (2, 2, 16, 5003, 1024, 4, "host", True),
+    (3, 3, 1, 9001, 2048, 16, "host", False), (2, 2, 4, 40000, 16384, 8, "host", False),
+    (2, 8, 4, 6000, 1024, 8, "device", False), (1, 2, 16, 20011, 2048, 16, "device", True),
+    (16, 8, 4, 6000, 4096, 8, "host", False)])
+def test_decode_equals_begin_and_end(gpu, B, H, G, ctx, budget, chunk, store, glm):
+    _say(f"decode chain B={B} H={H} G={G} ctx={ctx} budget={budget} chunk={chunk} {store} glm={glm}")
+    D, steps = 128, 4
+    table = (build_glm_cos_sin_cache(ctx + 64, 10000.0, device=gpu) if glm
+             else build_cos_sin_cache(ctx + 64, 500000.0, D, device=gpu))
+    cfg = types.SimpleNamespace(num_attention_heads=H * G, num_key_value_heads=H, hidden_size=H * G * D,
+                                num_hidden_layers=1)
+    g = torch.Generator(device=gpu).manual_seed(ctx)
+    base = torch.randn(B, H * G, 1, D, generator=g, device=gpu)
+    qs = [(0.95 * base + 0.3 * torch.randn(B, H * G, 1, D, generator=g, device=gpu)).to(torch.bfloat16)
+          for _ in range(steps)]
+    kv = [torch.randn(2, B, H, 1, D, generator=g, device=gpu).to(torch.bfloat16) for _ in range(steps)]
+    half = build_cos_sin_cache(ctx + 64, 500000.0, D, device=gpu)
+
+    def rope(q, k, pos):
+        return (apply_rotary_pos_emb_cuda(q, half, pos.expand(B, H * G, 1)),
+                apply_rotary_pos_emb_cuda(k, half, pos.expand(B, H, 1)))
+
+    got = []
+    for joined in (True, False):
+        cache = ShadowKVCache_CPU(cfg, batch_size=B, max_length=ctx, device=str(gpu), sparse_budget=budget,
+                                  chunk_size=chunk, rank=64, max_decode_len=steps, value_store=store)
+        synthesize_state(cache, ctx, seed=7, cos_sin=table)
+        attn = ShadowAttention(cache, G, D, H * G * D, rope, None, table)
+        outs = []
+        for i in range(steps):
+            pos = torch.full((1, 1, 1), ctx + i, dtype=torch.int64, device=gpu)
+            args = (qs[i], kv[i][0], kv[i][1], pos, 0)
+            out = attn.decode(*args) if joined else attn.decode_end(attn.decode_begin(*args))
+            live = cache.sparse_end + cache.gen_offset
+            v = cache.v_cache_buffer[0, :, :, :live].clone()
+            if store == "device":  # (read in place: the selected region of the value buffer is not kept)
+                v[:, :, cache.sparse_start:cache.sparse_end] = 0
+            outs.append([out.clone(), cache.position_ids.clone(), cache.cnts.clone(),
+                         cache.k_cache_buffer[0, :, :, :live].clone(), v])
+        torch.cuda.synchronize()
+        got.append(outs)
+        del cache, attn
+    for i in range(steps):
+        for a, b, what in zip(got[0][i], got[1][i], ("output", "position_ids", "hits", "keys", "values")):
+            assert torch.equal(a, b), (i, what)
+    assert any(0 < int(x[2].max()) for x in got[0][1:]), "no cache hits: the moves were not exercised"
