@@ -31,30 +31,43 @@ __device__ __forceinline__ u32x4 pack8(const float* f) {
   return u32x4{skv::f2bf2(f[0], f[1]), skv::f2bf2(f[2], f[3]), skv::f2bf2(f[4], f[5]), skv::f2bf2(f[6], f[7])};
 }
 
-// One workgroup per row; each thread owns 8-element vectors strided by the workgroup.
+// One workgroup per row; each thread owns 8-element vectors strided by the workgroup. Bound by
+// latency (8 KB rows, a few workgroups): one trip to memory, the weights requested with the row and
+// not after the reduction, and one vector per thread up to 4096 elements.
+constexpr int kNormThreads = 512;
+
 template <bool kResidual>
-__global__ void __launch_bounds__(kThreads) rmsnorm_kernel(const uint16_t* __restrict__ x, int64_t xs,
-                                                           const uint16_t* __restrict__ r, int64_t rs,
-                                                           uint16_t* __restrict__ ro, int64_t ros,
-                                                           const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
-                                                           int64_t os, int hidden, float eps) {
-  constexpr int kMaxVec = 4;  // hidden <= 4 * 8 * 256 = 8192
-  __shared__ float part[kThreads / 64];
+__global__ void __launch_bounds__(kNormThreads) rmsnorm_kernel(const uint16_t* __restrict__ x, int64_t xs,
+                                                               const uint16_t* __restrict__ r, int64_t rs,
+                                                               uint16_t* __restrict__ ro, int64_t ros,
+                                                               const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
+                                                               int64_t os, int hidden, float eps) {
+  constexpr int kMaxVec = 2;  // hidden <= 2 * 8 * 512 = 8192
+  __shared__ float part[kNormThreads / 64];
   const int row = blockIdx.x;
   const int nv = hidden / 8;
+  u32x4 xv[kMaxVec], rv[kMaxVec], wv[kMaxVec];
+#pragma unroll
+  for (int k = 0; k < kMaxVec; ++k) {
+    const int v = threadIdx.x + k * kNormThreads;
+    if (v < nv) {
+      xv[k] = *reinterpret_cast<const u32x4*>(x + row * xs + 8 * v);
+      if (kResidual) rv[k] = *reinterpret_cast<const u32x4*>(r + row * rs + 8 * v);
+      wv[k] = *reinterpret_cast<const u32x4*>(w + 8 * v);
+    }
+  }
   float h[kMaxVec][8];
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < kMaxVec; ++k) {
-    const int v = threadIdx.x + k * kThreads;
+    const int v = threadIdx.x + k * kNormThreads;
     if (v < nv) {
-      const u32x4 xv = *reinterpret_cast<const u32x4*>(x + row * xs + 8 * v);
-      unpack8(xv, h[k]);
+      unpack8(xv[k], h[k]);
       if (kResidual) {
-        float rv[8];
-        unpack8(*reinterpret_cast<const u32x4*>(r + row * rs + 8 * v), rv);
+        float f[8];
+        unpack8(rv[k], f);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) h[k][e] = skv::bf2f(skv::f2bf(h[k][e] + rv[e]));  // bf16 residual add
+        for (int e = 0; e < 8; ++e) h[k][e] = skv::bf2f(skv::f2bf(h[k][e] + f[e]));  // bf16 residual add
         *reinterpret_cast<u32x4*>(ro + row * ros + 8 * v) = pack8(h[k]);
       }
 #pragma unroll
@@ -66,16 +79,16 @@ __global__ void __launch_bounds__(kThreads) rmsnorm_kernel(const uint16_t* __res
   __syncthreads();
   float tot = 0.f;
 #pragma unroll
-  for (int i = 0; i < kThreads / 64; ++i) tot += part[i];
+  for (int i = 0; i < kNormThreads / 64; ++i) tot += part[i];
   const float inv = rsqrtf(tot / static_cast<float>(hidden) + eps);
 #pragma unroll
   for (int k = 0; k < kMaxVec; ++k) {
-    const int v = threadIdx.x + k * kThreads;
+    const int v = threadIdx.x + k * kNormThreads;
     if (v < nv) {
-      float wv[8], y[8];
-      unpack8(*reinterpret_cast<const u32x4*>(w + 8 * v), wv);
+      float f[8], y[8];
+      unpack8(wv[k], f);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = h[k][e] * inv * wv[e];
+      for (int e = 0; e < 8; ++e) y[e] = h[k][e] * inv * f[e];
       *reinterpret_cast<u32x4*>(out + row * os + 8 * v) = pack8(y);
     }
   }
@@ -181,10 +194,10 @@ extern "C" int skv_rmsnorm(const uint16_t* x, int64_t x_stride, const uint16_t* 
   }
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (residual)
-    hipLaunchKernelGGL(rmsnorm_kernel<true>, dim3(rows), dim3(kThreads), 0, s, x, x_stride, residual, residual_stride,
+    hipLaunchKernelGGL(rmsnorm_kernel<true>, dim3(rows), dim3(kNormThreads), 0, s, x, x_stride, residual, residual_stride,
                        residual_out, residual_out_stride, weight, out, out_stride, hidden, eps);
   else
-    hipLaunchKernelGGL(rmsnorm_kernel<false>, dim3(rows), dim3(kThreads), 0, s, x, x_stride, residual, residual_stride,
+    hipLaunchKernelGGL(rmsnorm_kernel<false>, dim3(rows), dim3(kNormThreads), 0, s, x, x_stride, residual, residual_stride,
                        residual_out, residual_out_stride, weight, out, out_stride, hidden, eps);
   return skv_check_launch(what);
 }

@@ -216,6 +216,7 @@ class ShadowKVCache_CPU(KVCacheBase):
         # Device-resident append row / attention length (use_device_lengths); None = host integers.
         self.append_row_dev = None
         self.kv_len_dev = None
+        self._lengths = torch.zeros(2, dtype=torch.int64)  # (both, once they are on the device)
         # Chunk pool tables (allocated with the prompt geometry) and per-step scratch.
         self.slot_of = self.slot_chunk = self.slot_used = self.pool_clock = None
         if self.pooled:
@@ -667,9 +668,20 @@ class ShadowKVCache_CPU(KVCacheBase):
         advances itself (at layer 0), so a whole step can be captured in a HIP graph and replayed.
         The host counters stay authoritative for the capacity check."""
         row = self.sparse_end + self.gen_offset - 1  # advanced before the step's first append
-        # physical append row (after the pool's extra slots); the attention length stays virtual
-        self.append_row_dev = torch.full((1,), row + self.pool_delta, dtype=torch.int64, device=self.device)
-        self.kv_len_dev = torch.full((1,), row + 1, dtype=torch.int32, device=self.device)
+        # physical append row (after the pool's extra slots); the attention length stays virtual. Two
+        # words of one tensor, the length (int32) the low half of the second: one launch advances both.
+        self._lengths = torch.full((2,), row + 1, dtype=torch.int64, device=self.device)
+        self._lengths[:1].fill_(row + self.pool_delta)
+        self.append_row_dev = self._lengths[:1]
+        self.kv_len_dev = self._lengths.view(torch.int32)[2:3]
+
+    def _advance_device_lengths(self):
+        base = self._lengths.data_ptr()
+        if self.append_row_dev.data_ptr() == base and self.kv_len_dev.data_ptr() == base + 8:
+            self._lengths.add_(1)
+        else:  # (a caller's own tensors)
+            self.append_row_dev.add_(1)
+            self.kv_len_dev.add_(1)
 
     def rope_and_append(self, qkv: torch.Tensor, position_ids: torch.Tensor, cos_sin: torch.Tensor, layer_idx: int,
                         q_out: torch.Tensor) -> torch.Tensor:
@@ -681,8 +693,7 @@ class ShadowKVCache_CPU(KVCacheBase):
             raise RuntimeError("rope_and_append needs use_device_lengths()")
         self.check_capacity(1)
         if layer_idx == 0:
-            self.append_row_dev.add_(1)
-            self.kv_len_dev.add_(1)
+            self._advance_device_lengths()
         shadowkv.rope_qk_append(qkv, self.num_attention_heads, self.num_key_value_heads, position_ids, cos_sin, q_out,
                                 self.k_cache_buffer[layer_idx], self.v_cache_buffer[layer_idx], self.append_row_dev)
         if layer_idx == self.num_layers - 1:
@@ -699,8 +710,7 @@ class ShadowKVCache_CPU(KVCacheBase):
             raise RuntimeError("qkv_rope_and_append needs use_device_lengths()")
         self.check_capacity(1)
         if layer_idx == 0:
-            self.append_row_dev.add_(1)
-            self.kv_len_dev.add_(1)
+            self._advance_device_lengths()
         shadowkv.linear_qkv_rope_append(x, wqkv_rope, self.num_attention_heads, self.num_key_value_heads,
                                         position_ids, cos_sin, q_out, self.k_cache_buffer[layer_idx],
                                         self.v_cache_buffer[layer_idx], self.append_row_dev, bias_rope)
@@ -715,8 +725,7 @@ class ShadowKVCache_CPU(KVCacheBase):
             if incoming != 1:
                 raise ValueError("device-resident lengths advance one token per decode step")
             if layer_idx == 0:
-                self.append_row_dev.add_(1)
-                self.kv_len_dev.add_(1)
+                self._advance_device_lengths()
             self.v_cache_buffer[layer_idx].index_copy_(2, self.append_row_dev, new_v_cache)
             self.k_cache_buffer[layer_idx].index_copy_(2, self.append_row_dev, new_k_cache)
         else:
