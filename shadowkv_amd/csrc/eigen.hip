@@ -6,7 +6,7 @@
 //                    scheme, Golub & Van Loan 8.3.1). The matrix stays in registers, 8 columns per
 //                    wave, the waves of one problem on the CUs of one XCD.
 //   bisect_kernel    the R largest eigenvalues of T: Sturm counts in fp64 (the number of sign changes
-//                    of the leading principal minors), one wave per eigenvalue, 64 points per pass.
+//                    of the leading principal minors), one workgroup per eigenvalue.
 //   (in it)          their eigenvectors from T by a twisted factorisation in fp64 (Dhillon & Parlett):
 //                    forward and backward pivots, joined where the twisted pivot is smallest.
 //   backtransform    Q times each vector, one wave per vector.
@@ -21,8 +21,8 @@
 // all), the polling loads agent-scope (past the L1). Every wait is bounded: a workgroup that waits too long
 // gives up for good, the problem's status says so and the caller takes another way.
 //
-// MI355X, rank 160, us in all: n = 1024 2290 (the reduction 1640, 1.6 a step; the eigenpairs of T 460; the
-// back transformation 180), n = 512 909, n = 256 416 (1.0 a step: the exchange and the chain of
+// MI355X, rank 160, us in all: n = 1024 2190 (the reduction 1640, 1.6 a step; the eigenpairs of T 360; the
+// back transformation 180), n = 512 848, n = 256 386 (1.0 a step: the exchange and the chain of
 // reductions alone); rocSOLVER's full decomposition 19600, 10400, 4900.
 #include <type_traits>
 
@@ -314,16 +314,26 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
   return v;
 }
 
-// One wave per eigenpair of T: eigenvalue k of the descending order, then its vector.
-__global__ void __launch_bounds__(64) bisect_kernel(EigenArgs g, int npad) {
-  const int b = blockIdx.y, k = blockIdx.x, n = g.n, lane = threadIdx.x;
+// One workgroup per eigenpair of T: eigenvalue k of the descending order, then its vector. Bound by the
+// chain of n fp64 recurrence steps of every pass, so a pass takes as many points as run beside one
+// another without slowing the chain (one wave per SIMD): 256 points in 7 passes, where one wave took 9
+// passes of 64. The pivots of the twisted factorisation are quotients of neighbouring minors, taken in
+// parallel after the same two-term recurrence: dividing along the chain cost five times as much.
+constexpr int kPoints = 256;
+constexpr int kPointWaves = kPoints / 64;
+
+__global__ void __launch_bounds__(kPoints) bisect_kernel(EigenArgs g, int npad) {
+  const int b = blockIdx.y, k = blockIdx.x, n = g.n, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (g.status[b] != 1) return;
+  __shared__ double red[2][kPointWaves];
+  __shared__ int votes[2][kPointWaves];
   __shared__ double2 de[kMaxN];  // diagonal, square of the off-diagonal before it
-  __shared__ double es[kMaxN], q[2][kMaxN];
+  __shared__ double es[kMaxN], q0[kMaxN], q1[kMaxN];  // pivots from the front and from the back
+  __shared__ double2 pp[2][kMaxN];                     // minors: (p, the one before it), in one scale
   const float* d = g.d + b * npad;
   const float* e = g.e + b * npad;
   double lo = 1e300, hi = -1e300;  // Gershgorin
-  for (int i = lane; i < n; i += 64) {
+  for (int i = tid; i < n; i += kPoints) {
     const double di = d[i], ei = i + 1 < n ? e[i] : 0.f, em = i > 0 ? e[i - 1] : 0.f;
     de[i] = make_double2(di, em * em);
     es[i] = ei;
@@ -336,71 +346,120 @@ __global__ void __launch_bounds__(64) bisect_kernel(EigenArgs g, int npad) {
     lo = fmin(lo, __shfl_xor(lo, o, 64));
     hi = fmax(hi, __shfl_xor(hi, o, 64));
   }
+  if (lane == 0) {
+    red[0][wave] = lo;
+    red[1][wave] = hi;
+  }
   __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPointWaves; ++i) {
+    lo = fmin(lo, red[0][i]);
+    hi = fmax(hi, red[1][i]);
+  }
   const double norm = fmax(fabs(lo), fabs(hi));
   lo -= 1e-12 * norm;
   hi += 1e-12 * norm;
-  // 64 interior points split [lo, hi] into 65 parts; lambda_k >= x when at least k + 1 eigenvalues are
+  // Past n up to a multiple of 8: a factor that changes neither sign nor count.
+  const int n8 = (n + 7) / 8 * 8;
+  for (int i = n + tid; i < n8; i += kPoints) de[i] = make_double2(hi + norm, 0.0);
+  __syncthreads();
+  auto rescale = [](double& p0, double& p1) {  // (powers of two would do; only the ratio matters)
+    const double m = fmax(fabs(p0), fabs(p1));
+    const double f = m > 1e100 ? 1e-100 : m < 1e-100 ? 1e100 : 1.0;
+    p0 *= f;
+    p1 = m == 0.0 ? 1e-100 : p1 * f;
+  };
+  // The interior points split [lo, hi] into 257 parts; lambda_k >= x when at least k + 1 eigenvalues are
   // not below x, and the eigenvalues below x are the sign changes of the minors p_i (an exact zero
-  // between two nonzero minors counts once with either sign). 9 passes: 65^-9 of the
-  // width (8, 3e-15, are not enough for the vectors of a spectrum that ends in rounding noise).
-  for (int pass = 0; pass < 9; ++pass) {
-    const double step = (hi - lo) / 65.0;
-    const double x = lo + step * (lane + 1);
+  // between two nonzero minors counts once with either sign). 7 passes: 257^-7 = 1e-17 of the width
+  // (3e-15 is not enough for the vectors of a spectrum that ends in rounding noise).
+  for (int pass = 0; pass < 7; ++pass) {
+    const double step = (hi - lo) / (kPoints + 1);
+    const double x = lo + step * (tid + 1);
     double p0 = 0.0, p1 = 1.0;
     int below = 0;
-    auto advance = [&](int i) {
-      const double2 t = de[i];
-      const double p = fma(t.x - x, p1, -t.y * p0);
-      below += static_cast<int>(static_cast<uint32_t>(__double2hiint(p) ^ __double2hiint(p1)) >> 31);
-      p0 = p1;
-      p1 = p;
-    };
-    int i = 0;
-    for (; i < n; i += 8) {
-      if (i + 8 <= n) {
+    // Eight steps at a time, the next eight's coefficients requested ahead (read as they are needed,
+    // their LDS latency is half of a step).
+    double2 next[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) advance(i + u);
-      } else {
-        for (int u = i; u < n; ++u) advance(u);
+    for (int u = 0; u < 8; ++u) next[u] = de[u];
+    for (int i = 0; i < n8; i += 8) {
+      double2 t[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) t[u] = next[u];
+      const int ahead = min(i + 8, n8 - 8);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) next[u] = de[ahead + u];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const double p = fma(t[u].x - x, p1, -t[u].y * p0);
+        below += static_cast<int>(static_cast<uint32_t>(__double2hiint(p) ^ __double2hiint(p1)) >> 31);
+        p0 = p1;
+        p1 = p;
       }
-      const double m = fmax(fabs(p0), fabs(p1));
-      const double f = m > 1e100 ? 1e-100 : m < 1e-100 ? 1e100 : 1.0;
-      p0 *= f;
-      p1 = m == 0.0 ? 1e-100 : p1 * f;
+      rescale(p0, p1);
     }
-    // Lanes' points ascend: those at most lambda_k form a prefix.
-    const int c = __popcll(__ballot(n - below >= k + 1));
-    const double nlo = c > 0 ? lo + step * c : lo, nhi = c < 64 ? lo + step * (c + 1) : hi;
+    // The threads' points ascend: those at most lambda_k form a prefix.
+    const int mine = __popcll(__ballot(n - below >= k + 1));
+    if (lane == 0) votes[pass & 1][wave] = mine;
+    __syncthreads();
+    int c = 0;
+#pragma unroll
+    for (int i = 0; i < kPointWaves; ++i) c += votes[pass & 1][i];
+    const double nlo = c > 0 ? lo + step * c : lo, nhi = c < kPoints ? lo + step * (c + 1) : hi;
     lo = nlo;
     hi = nhi;
   }
   const double lam = 0.5 * (lo + hi);
-  // Pivots from both ends: lane 0 forward, lane 1 backward.
-  const double tiny = 1e-18 * norm * 1e-12 + 1e-300;
-  if (lane < 2) {
-    double qq = 0.0;
-#pragma unroll 4
-    for (int t = 0; t < n; ++t) {
-      const int i = lane ? n - 1 - t : t;
-      const double ee = t == 0 ? 0.0 : lane ? es[i] : es[i - 1];
-      double nq = de[i].x - lam;
-      if (t > 0) {
-        double r = __builtin_amdgcn_rcp(qq);  // refined by two Newton steps
-        r = fma(fma(-qq, r, 1.0), r, r);
-        r = fma(fma(-qq, r, 1.0), r, r);
-        nq = fma(-ee * ee, r, nq);
+  // Minors from both ends: thread 0 forward, thread 1 backward. An exact zero becomes a tiny pivot.
+  const double tiny = 1e-30 * norm + 1e-300;
+  if (tid < 2) {
+    double p0 = 0.0, p1 = 1.0;
+    double2* out = pp[tid];
+    auto coef = [&](int t) {  // of the t-th step: diagonal, square of the off-diagonal before it
+      const int i = tid ? n - 1 - t : t;
+      const double e2 = tid ? es[i] * es[i] : de[i].y;
+      return make_double2(de[i].x - lam, t == 0 ? 0.0 : e2);
+    };
+    auto advance = [&](int t, const double2& c) {
+      double p = fma(c.x, p1, -c.y * p0);
+      if (p == 0.0) p = -tiny * p1;
+      out[tid ? n - 1 - t : t] = make_double2(p, p1);
+      p0 = p1;
+      p1 = p;
+    };
+    int t = 0;
+    if (n >= 8) {
+      double2 next[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) next[u] = coef(u);
+      for (; t + 8 <= n; t += 8) {
+        double2 c[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) c[u] = next[u];
+        const int ahead = min(t + 8, n - 8);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) next[u] = coef(ahead + u);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) advance(t + u, c[u]);
+        rescale(p0, p1);
       }
-      if (fabs(nq) < tiny) nq = -tiny;
-      q[lane][i] = nq;
-      qq = nq;
     }
+    for (; t < n; ++t) advance(t, coef(t));
+  }
+  __syncthreads();
+  for (int i = tid; i < n; i += kPoints) {
+    double f = pp[0][i].x / pp[0][i].y, r = pp[1][i].x / pp[1][i].y;
+    q0[i] = fabs(f) < tiny ? -tiny : f;
+    q1[i] = fabs(r) < tiny ? -tiny : r;
   }
   __syncthreads();
   double best = 1e300;
   int at = 0;
-  for (int i = lane; i < n; i += 64) {
-    const double gm = fabs(q[0][i] + q[1][i] - (de[i].x - lam));
+  for (int i = tid; i < n; i += kPoints) {
+    const double gm = fabs(q0[i] + q1[i] - (de[i].x - lam));
     if (gm < best) {
       best = gm;
       at = i;
@@ -415,31 +474,63 @@ __global__ void __launch_bounds__(64) bisect_kernel(EigenArgs g, int npad) {
       at = oa;
     }
   }
-  // Ratios of neighbouring entries, then their running products away from the twist.
-  for (int i = lane; i < n; i += 64) {
-    const double up = i + 1 < n ? -es[i] / q[0][i] : 0.0;    // z[i] / z[i + 1], i < at
-    const double dn = i > 0 ? -es[i - 1] / q[1][i] : 0.0;    // z[i] / z[i - 1], i > at
-    q[0][i] = i < at ? up : i > at ? dn : 1.0;
+  if (lane == 0) {
+    red[0][wave] = best;
+    votes[0][wave] = at;
   }
   __syncthreads();
-  if (lane < 2) {
-    double z = 1.0;
-    const int steps = lane ? n - 1 - at : at, dir = lane ? 1 : -1;
-#pragma unroll 8
-    for (int t = 1; t <= steps; ++t) {
-      z *= q[0][at + dir * t];
-      q[1][at + dir * t] = z;
+#pragma unroll
+  for (int i = 0; i < kPointWaves; ++i) {
+    const double ob = red[0][i];
+    const int oa = votes[0][i];
+    if (ob < best || (ob == best && oa < at)) {
+      best = ob;
+      at = oa;
     }
-    if (lane == 0) q[1][at] = 1.0;
+  }
+  // Ratios of neighbouring entries, then their running products away from the twist.
+  for (int i = tid; i < n; i += kPoints) {
+    const double up = i + 1 < n ? -es[i] / q0[i] : 0.0;   // z[i] / z[i + 1], i < at
+    const double dn = i > 0 ? -es[i - 1] / q1[i] : 0.0;   // z[i] / z[i - 1], i > at
+    q0[i] = i < at ? up : i > at ? dn : 1.0;
+  }
+  __syncthreads();
+  double* zz = q1;
+  if (tid < 2) {
+    double z = 1.0;
+    const int steps = tid ? n - 1 - at : at, dir = tid ? 1 : -1;
+    const double* src = q0 + at;
+    double* dst = zz + at;
+    int t = 1;
+    for (; t + 8 <= steps + 1; t += 8) {
+      double r[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) r[u] = src[dir * (t + u)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        z *= r[u];
+        dst[dir * (t + u)] = z;
+      }
+    }
+    for (; t <= steps; ++t) {
+      z *= src[dir * t];
+      dst[dir * t] = z;
+    }
+    if (tid == 0) zz[at] = 1.0;
   }
   __syncthreads();
   double ss = 0.0;
-  for (int i = lane; i < n; i += 64) ss = fma(q[1][i], q[1][i], ss);
+  for (int i = tid; i < n; i += kPoints) ss = fma(zz[i], zz[i], ss);
   ss = wave_sum_f64(ss);
+  if (lane == 0) red[1][wave] = ss;
+  __syncthreads();
+  ss = 0.0;
+#pragma unroll
+  for (int i = 0; i < kPointWaves; ++i) ss += red[1][i];
   const double inv = 1.0 / sqrt(ss);
   float* z = g.z + (static_cast<int64_t>(b) * g.rank + k) * npad;
-  for (int i = lane; i < npad; i += 64) z[i] = i < n ? static_cast<float>(q[1][i] * inv) : 0.f;
-  if (lane == 0) g.w[b * g.rank + k] = static_cast<float>(lam * static_cast<double>(g.scale[b]));
+  for (int i = tid; i < npad; i += kPoints) z[i] = i < n ? static_cast<float>(zz[i] * inv) : 0.f;
+  if (tid == 0) g.w[b * g.rank + k] = static_cast<float>(lam * static_cast<double>(g.scale[b]));
 }
 
 // vt[k] = H_0 H_1 ... H_{n-2} z_k, one wave per vector, the reflections requested kAhead steps ahead in
@@ -560,7 +651,7 @@ extern "C" int skv_sym_eig_top(const float* a, int batch, int n, int rank, float
   auto run = [&](auto nrv) {
     constexpr int NR = decltype(nrv)::value;
     hipLaunchKernelGGL(tridiag_kernel<NR>, dim3(256), dim3(kWgWaves * 64), 0, s, g);
-    hipLaunchKernelGGL(bisect_kernel, dim3(rank, batch), dim3(64), 0, s, g, 64 * NR);
+    hipLaunchKernelGGL(bisect_kernel, dim3(rank, batch), dim3(kPoints), 0, s, g, 64 * NR);
     hipLaunchKernelGGL(backtransform_kernel<NR>, dim3(rank, batch), dim3(64), 0, s, g);
   };
   if (nr == 2) run(std::integral_constant<int, 2>{});
