@@ -64,8 +64,18 @@ class ShadowAttention(AttentionBase):
         kv_cache = self.kv_cache
         kv_cache.get_svd(key_states, layer_idx=layer_idx)
         query_states, key_states = self.apply_rotary_pos_emb(query_states, key_states, position_ids)
-        kv_cache.prefill_kv_cache(value_states, layer_idx, key_states, query_states[:, :, -1:])
-        return causal_attention_fp32(query_states, key_states, value_states)
+        # The values' copy to the host runs beside the attention, and the attention's launch comes before
+        # the state's many small ones, whose issue by the host it covers (MI355X, one layer: 8192
+        # tokens on 8 kv heads 4.17 -> 3.74 ms, 19333 on 2 7.14 -> 6.51 ms).
+        copy = kv_cache._value_copy = kv_cache.start_value_copy(value_states, layer_idx)
+        try:
+            out = causal_attention_fp32(query_states, key_states, value_states)
+            kv_cache.prefill_kv_cache(value_states, layer_idx, key_states, query_states[:, :, -1:])
+        finally:
+            kv_cache._value_copy = None
+            if copy is not None:
+                copy.synchronize()
+        return out
 
     def decode(self, query_states, key_states, value_states, position_ids, layer_idx):
         """One new token through the layer: decode_begin() and decode_end(). Nothing can overlap the

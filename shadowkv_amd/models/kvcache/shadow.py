@@ -40,8 +40,8 @@ from .base import KVCacheBase
 
 def _top_eigenpairs(gram: torch.Tensor, rank: int):
     """The `rank` leading eigenpairs (w [b, rank] descending, vt [b, rank, n]) of the Gram matrices from
-    shadowkv.sym_eig_top, or None where it does not apply or its result does not hold up: residuals and
-    orthogonality within a few times what rocSOLVER's eigh shows on such matrices (residual 1 to 6e-7 of the
+    shadowkv.sym_eig_top and, still on the device, whether they hold up, or None where it does not
+    apply. Residuals and orthogonality are held to a few times what rocSOLVER's eigh shows on such matrices (residual 1 to 6e-7 of the
     largest eigenvalue, orthogonality 1 to 2.3e-6; the kernel's own: 0.8 to 1.8e-7 and 0.2 to 0.9e-6)."""
     b, n, _ = gram.shape
     if not (plain_eager(gram) and gram.dtype == torch.float32 and 64 <= n <= shadowkv.SYM_EIG_MAX_N and 1 <= rank <= n
@@ -57,9 +57,7 @@ def _top_eigenpairs(gram: torch.Tensor, rank: int):
             good.append((status == 1) & (res <= 2e-6 * w[:, 0]) & (orth <= 5e-6))
             ws.append(w)
             vts.append(vt)
-    if not bool(torch.cat(good).all()):
-        return None
-    return torch.cat(ws), torch.cat(vts)
+    return torch.cat(ws), torch.cat(vts), torch.cat(good).all()
 
 
 def low_rank_factors(k: torch.Tensor, rank: int):
@@ -74,7 +72,7 @@ def low_rank_factors(k: torch.Tensor, rank: int):
     kf = k.float()
     gram = torch.matmul(kf.transpose(1, 2), kf)
     top = _top_eigenpairs(gram, rank)
-    if top is None:
+    if top is None or not bool(top[2]):
         w, v = torch.linalg.eigh(gram)  # ascending eigenvalues
         w, v = w.flip(-1)[..., :rank], v.flip(-1)[..., :rank]
     else:
@@ -213,6 +211,7 @@ class ShadowKVCache_CPU(KVCacheBase):
         self.attn_workspace = None
         self.attn_out = None
         self.select_workspace = None  # allocated with the landmarks
+        self._value_copy = None  # a value copy started for the next prefill_kv_cache (its event)
         # Device-resident append row / attention length (use_device_lengths); None = host integers.
         self.append_row_dev = None
         self.kv_len_dev = None
@@ -258,8 +257,10 @@ class ShadowKVCache_CPU(KVCacheBase):
             with torch.cuda.device(keys.device):
                 top = _top_eigenpairs(shadowkv.keys_gram(keys), R)
                 if top is not None:
-                    shadowkv.keys_factors(keys, *top, U, SV)
-                    return
+                    # (the factors are launched before the host waits for the verdict, which is hardly ever no)
+                    shadowkv.keys_factors(keys, top[0], top[1], U, SV)
+                    if bool(top[2]):
+                        return
         k = new_k_cache.transpose(1, 2).reshape(bsz, -1, H * D) if new_k_cache.shape[1] <= 32 else new_k_cache
         u, svt = low_rank_factors(k, R)
         U.copy_(u.to(self.dtype))
@@ -332,6 +333,33 @@ class ShadowKVCache_CPU(KVCacheBase):
         shadowkv.gather_copy_with_offsets(src_chunks, dst, None, offs, cnts, None, bsz, H, nch * c * D, m * c * D,
                                           start_row * D, self.buf_len * D, m, misses_only=True)
 
+    def start_value_copy(self, new_v_cache: torch.Tensor, layer_idx: int):
+        """Begins the copy of a prompt's value chunks to the layer's pinned host store on the fetch stream,
+        beside the work that follows on the current one. Returns the event that prefill_kv_cache waits for
+        on the host, or None where prefill_kv_cache makes the copy itself: a store in device memory, values
+        whose rows are not contiguous, tracing. A caller that starts the copy of a prompt's values early
+        leaves the event in _value_copy for the prefill_kv_cache call on the same values."""
+        bsz, H, incoming, D = new_v_cache.shape
+        c, pb = self.chunk_size, self.prefilled_batch
+        n = incoming // c
+        store = self.v_cache_cpu[layer_idx]
+        v = new_v_cache
+        if not (self.value_store == "host" and plain_eager(v) and v.dtype == store.dtype and v.stride(-1) == 1
+                and v.stride(-2) == D and 0 < n <= store.shape[2] and pb + bsz <= store.shape[0] and bsz * H <= 64
+                and not torch.cuda.is_current_stream_capturing()):
+            return None
+        dst = store[pb:pb + bsz, :, :n]
+        src = v[:, :, :n * c]
+        self.copy_stream.wait_stream(torch.cuda.current_stream(v.device))
+        with torch.cuda.stream(self.copy_stream):
+            if dst.is_contiguous() and src.is_contiguous():
+                dst.copy_(src.view(dst.shape), non_blocking=True)
+            else:  # row by row: torch would stage a strided destination through pageable memory
+                for b in range(bsz):
+                    for h in range(H):
+                        dst[b, h].copy_(src[b, h].view(n, c * D), non_blocking=True)
+            return self.copy_stream.record_event()
+
     def prefill_kv_cache(self, new_v_cache: torch.Tensor, layer_idx: int, key_states_roped: torch.Tensor,
                          last_query_states: torch.Tensor = None):
         """Build one layer's decode state from the prefill K/V (shadow.py:463-544), on the device:
@@ -349,8 +377,23 @@ class ShadowKVCache_CPU(KVCacheBase):
         v = new_v_cache if new_v_cache.stride(-1) == 1 and new_v_cache.stride(-2) == D else new_v_cache.contiguous()
         k = key_states_roped if key_states_roped.stride(-1) == 1 and key_states_roped.stride(-2) == D \
             else key_states_roped.contiguous()
-        self.v_cache_cpu[l][pb:pb + bsz, :, :max_ctx_chunks].copy_(
-            v[:, :, :self.max_ctx_chunks_len].reshape(bsz, H, max_ctx_chunks, c * D))
+        value_copy, self._value_copy = self._value_copy, None
+        if value_copy is None:
+            value_copy = self.start_value_copy(v, l)
+        if value_copy is None:
+            self.v_cache_cpu[l][pb:pb + bsz, :, :max_ctx_chunks].copy_(
+                v[:, :, :self.max_ctx_chunks_len].reshape(bsz, H, max_ctx_chunks, c * D))
+        try:
+            self._encode_layer(k, v, l, last_query_states)
+        finally:
+            if value_copy is not None:  # the host store is whole when this returns (and v may be freed)
+                value_copy.synchronize()
+        self._finish_layer(l, bsz, incoming)
+
+    def _encode_layer(self, k: torch.Tensor, v: torch.Tensor, l: int, last_query_states: torch.Tensor):
+        """The device part of prefill_kv_cache: buffers, landmarks and the initial selection."""
+        bsz, H, incoming, D = v.shape
+        c, pb, G = self.chunk_size, self.prefilled_batch, self.num_key_value_groups
         kbuf = self.k_cache_buffer[l][pb:pb + bsz]
         vbuf = self.v_cache_buffer[l][pb:pb + bsz]
         kbuf[:, :, :self.prefill_local].copy_(k[:, :, -self.prefill_local:])
@@ -387,7 +430,6 @@ class ShadowKVCache_CPU(KVCacheBase):
         self._copy_chunks(v, vbuf, selected, self.sparse_start)
         self._copy_chunks(k, kbuf, selected, self.sparse_start)
         self.init_pool(l, pb, bsz)
-        self._finish_layer(l, bsz, incoming)
 
     def init_pool(self, layer_idx: int, pb: int = 0, bsz: int | None = None):
         """Pool tables of one layer from its initial selection: slot j holds position_ids[j]

@@ -97,3 +97,35 @@ def test_get_svd_routes(gpu, form, monkeypatch):
     assert diff < 4e-3, diff  # two bf16 roundings of the same fp32 factors, up to their signs
     err = (rec[0].reshape(B, ctx, -1) - k.double()).norm() / k.double().norm()
     assert err < 0.08  # the noise outside rank 64
+
+
+@pytest.mark.parametrize("ctx,max_length,B,first", [(1400, 1400, 2, 2), (1403, 2048, 2, 1), (1800, 4096, 3, 2)])
+def test_prefill_value_copy(gpu, ctx, max_length, B, first):
+    """The host store after prefill and prefill_kv_cache, from whole, ragged and padded rows and batches
+    prefilled in parts: every value chunk, nothing else; a transposed view of the values too."""
+    from shadowkv_amd.models.attention import ShadowAttention
+    from shadowkv_amd.models.tensor_op import build_cos_sin_cache
+    _say(f"value copy ctx={ctx} max={max_length} B={B} first={first}")
+    H, G, D, c = 2, 2, 128, 8
+    cfg = types.SimpleNamespace(num_attention_heads=G * H, num_key_value_heads=H, hidden_size=G * H * D,
+                                num_hidden_layers=1)
+    g = torch.Generator().manual_seed(ctx)
+    table = build_cos_sin_cache(max_length, 10000.0, D, device=gpu)
+    q, k, v = (torch.randn(B, h, ctx, D, generator=g).to(torch.bfloat16).to(gpu) for h in (G * H, H, H))
+    for form in ("prefill", "encode", "view"):
+        cache = ShadowKVCache_CPU(cfg, batch_size=B, max_length=max_length, device=str(gpu), sparse_budget=1024, rank=32)
+        attn = ShadowAttention(cache, G, D, G * H * D, lambda a, b, p: (a, b), None, table)
+        for lo, hi in ((0, first), (first, B)):
+            if lo == hi:
+                continue
+            vv = v[lo:hi] if form != "view" else v[lo:hi].transpose(1, 2).contiguous().transpose(1, 2)
+            if form == "prefill":
+                attn.prefill(q[lo:hi], k[lo:hi], vv, None, 0)
+            else:
+                cache.get_svd(k[lo:hi], 0)
+                cache.prefill_kv_cache(vv, 0, k[lo:hi], q[lo:hi, :, -1:])
+            n = ctx // c
+            got = cache.v_cache_cpu[0]  # (read at once: the call has waited for the copy)
+            assert torch.equal(got[lo:hi, :, :n], v[lo:hi, :, :n * c].reshape(hi - lo, H, n, c * D).cpu())
+            assert not got[:, :, n:].any() and not got[hi:].any()
+        del cache, attn
