@@ -445,6 +445,49 @@ def test_rebuild_tile_shapes_agree(gpu, glm, monkeypatch):
     torch.testing.assert_close(outs[0].float(), want.float(), rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("B,H,S,D,form", [(1, 1, 1, 16, "plain"), (2, 3, 37, 128, "plain"), (1, 5, 130, 128, "tokens"),
+                                          (2, 2, 9, 48, "odd"), (2, 3, 33, 128, "strided"), (1, 2, 5, 24, "plain")])
+def test_rope_new_forms(gpu, B, H, S, D, form):
+    """apply_rotary_pos_emb_new in its 16-byte and its scalar form (rows at an odd offset, a half that is not
+    a multiple of 8, dims strided): the same bits, NaN and infinities included, rows outside the table left."""
+    _say(f"rope new B={B} H={H} S={S} D={D} {form}")
+    g = torch.Generator().manual_seed(S * 10 + D)
+    rows = 50
+    x = torch.randn(B, H, S, D, generator=g).to(torch.bfloat16)
+    x[0, 0, 0, 0], x[0, 0, 0, 1], x[0, 0, 0, 2] = float("nan"), float("inf"), -0.0
+    cs = torch.randn(rows, D, generator=g).to(torch.bfloat16)
+    pos = torch.randint(0, rows, (B, H, S), generator=g)
+    if S > 4:
+        pos[0, 0, 3], pos[B - 1, H - 1, 4] = rows, -1
+    inside = (pos >= 0) & (pos < rows)
+    half = D // 2
+    c = cs[pos.clamp(0, rows - 1)]
+    x1, x2 = x[..., :half], x[..., half:]
+    want = torch.cat((x1 * c[..., :half] + (-x2) * c[..., half:], x2 * c[..., :half] + x1 * c[..., half:]), -1)
+    want = torch.where(inside.unsqueeze(-1), want, torch.full_like(want, 5.0))
+
+    def buf(fill):
+        if form == "tokens":
+            return torch.full((B, S, H, D), fill, dtype=torch.bfloat16, device=gpu).transpose(1, 2)
+        if form == "odd":
+            return torch.full((B * H * S * D + 1,), fill, dtype=torch.bfloat16, device=gpu)[1:].view(B, H, S, D)
+        if form == "strided":
+            return torch.full((B, H, S, 2 * D), fill, dtype=torch.bfloat16, device=gpu)[..., ::2]
+        return torch.full((B, H, S, D), fill, dtype=torch.bfloat16, device=gpu)
+
+    xd, out = buf(0.0), buf(5.0)
+    xd.copy_(x)
+    shadowkv.apply_rotary_pos_emb_new(xd, cs.to(gpu), pos.to(gpu), out, B, H, S, D, *xd.stride(), D, *pos.stride(), half)
+    torch.cuda.synchronize()
+    got = out.cpu()
+    nan = want.isnan()
+    assert torch.equal(got.isnan(), nan) and torch.equal(got[~nan], want[~nan])
+    # in place
+    shadowkv.apply_rotary_pos_emb_new(xd, cs.to(gpu), pos.to(gpu), xd, B, H, S, D, *xd.stride(), D, *pos.stride(), half)
+    keep = inside.unsqueeze(-1) & ~nan
+    assert torch.equal(xd.cpu()[keep.expand_as(x)], want[keep.expand_as(x)])
+
+
 def test_rope_two_tables_and_chunk_positions(gpu):
     """The reference's remaining rotary bindings: separate cos/sin tables (apply_rotary_pos_emb),
     chunk-id positions without hit rows (apply_rotary_pos_emb_new_v2), and push_cache (the _opt
