@@ -65,13 +65,12 @@ LANE_FETCH_WORKGROUPS = 64
 LANE_REBUILD_WORKGROUPS = 48
 
 
-# Token rows up to which the decoder's projections use the library's skinny linear kernel; above
-# it, torch's GEMM (hipBLASLt). Measured on MI355X with cold Llama-3-8B weights, µs per launch,
-# skinny vs hipBLASLt: 8 rows qkv 13.1 / 14.4, o_proj 10.8 / 15.8, gate_up 50.6 / 58.9, down
-# 26.6 / 26.7; 12 rows 29.0 / 14.3, 21.0 / 15.8, 125.3 / 59.5, 63.3 / 25.8; 16 rows 30.9 / 14.3,
-# 21.6 / 15.7, 132.6 / 59.5, 64.8 / 26.6 (the kernel's 9-16-row form streams two weight rows per
-# workgroup).
-SKINNY_LINEAR_ROWS = 8
+# Token rows up to which the decoder's projections use the library's skinny linear kernel (all that it
+# takes); above, torch's GEMM (hipBLASLt). Measured on MI355X with cold Llama-3-8B weights, µs per
+# launch, skinny vs hipBLASLt: 8 rows qkv 11.7 / 15.9, o_proj 8.4 / 13.5, gate_up 38.7 / 62.3, down 22.3 /
+# 26.7, head 159 / 187; 12 rows 12.7 / 15.9, 9.0 / 14.5, 41.3 / 62.0, 23.3 / 26.3, 172 / 188; 16 rows 13.3 /
+# 15.7, 9.2 / 14.3, 43.2 / 62.5, 24.6 / 26.9, 183 / 189.
+SKINNY_LINEAR_ROWS = 16
 
 
 def pool_miss_fraction(pool_slots: int | None, landmarks: int) -> float:
