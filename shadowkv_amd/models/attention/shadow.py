@@ -12,6 +12,7 @@ import math
 import torch
 
 from ...kernels import shadowkv
+from ..kvcache.shadow import ShadowKVCache_CPU
 from ..tensor_op import plain_eager, repeat_kv
 from .base import AttentionBase
 
@@ -58,6 +59,11 @@ def causal_attention_fp32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, blo
 JOINED_FETCH_WORKGROUPS = 128
 
 
+# The steps of decode_begin() that the joined chain of decode() does otherwise.
+_CACHE_STEPS = ("get_retrieval_position_ids", "get_value_cache", "get_key_cache", "move_value_hits")
+_ATTENTION_STEPS = ("decode_begin", "decode_begin_appended", "_key_path")
+
+
 class ShadowAttention(AttentionBase):
 
     def prefill(self, query_states, key_states, value_states, position_ids, layer_idx):
@@ -85,7 +91,7 @@ class ShadowAttention(AttentionBase):
         and two launches side by side (the same buffer contents). MI355X, values in host memory,
         one sequence of 8192 tokens: 236 -> 144 us, 4 of 122880: 287 -> 242 us."""
         kv_cache = self.kv_cache
-        if kv_cache.pooled or kv_cache.fold_hit_moves or getattr(kv_cache, "key_stream", None) is not None:
+        if not self._joined(kv_cache):
             return self.decode_end(self.decode_begin(query_states, key_states, value_states, position_ids, layer_idx))
         query_states, key_states = self.apply_rotary_pos_emb(query_states, key_states, position_ids)
         kv_cache.update_kv_cache(key_states, value_states, layer_idx)
@@ -94,6 +100,20 @@ class ShadowAttention(AttentionBase):
             layer_idx, position_ids, self.cos_sin_cache,
             fetch_workgroups=kv_cache.fused_fetch_workgroups or JOINED_FETCH_WORKGROUPS)
         return self.decode_end((query_states, key_states, value_states, [], layer_idx))
+
+    def _joined(self, kv_cache) -> bool:
+        """Whether decode() may take the joined chain: a cache in its default setting, and neither class's
+        steps of the two-stream chain replaced (they would not be called)."""
+        if kv_cache.pooled or kv_cache.fold_hit_moves or getattr(kv_cache, "key_stream", None) is not None:
+            return False
+        cache_type, own = type(kv_cache), vars(kv_cache)
+        if cache_type is not ShadowKVCache_CPU and any(
+                getattr(cache_type, n) is not getattr(ShadowKVCache_CPU, n) for n in _CACHE_STEPS):
+            return False
+        if type(self) is not ShadowAttention and any(
+                getattr(type(self), n) is not getattr(ShadowAttention, n) for n in _ATTENTION_STEPS):
+            return False
+        return not any(n in own for n in _CACHE_STEPS) and not any(n in vars(self) for n in _ATTENTION_STEPS)
 
     def decode_begin(self, query_states, key_states, value_states, position_ids, layer_idx):
         """First half of decode(): RoPE, append, chunk selection, the value fetch launched on the

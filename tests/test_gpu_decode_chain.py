@@ -66,3 +66,40 @@ def test_decode_equals_begin_and_end(gpu, B, H, G, ctx, budget, chunk, store, gl
         for a, b, what in zip(got[0][i], got[1][i], ("output", "position_ids", "hits", "keys", "values")):
             assert torch.equal(a, b), (i, what)
     assert any(0 < int(x[2].max()) for x in got[0][1:]), "no cache hits: the moves were not exercised"
+
+
+def test_replaced_steps_are_called(gpu):
+    """A cache or attention whose steps of the two-stream chain are replaced, on the instance or in a
+    subclass, keeps that chain."""
+    _say("decode chain replaced steps")
+    cfg = types.SimpleNamespace(num_attention_heads=8, num_key_value_heads=2, hidden_size=1024, num_hidden_layers=1)
+    table = build_cos_sin_cache(3000, 500000.0, 128, device=gpu)
+
+    class Counting(ShadowKVCache_CPU):
+        calls = 0
+
+        def get_key_cache(self, *args, **kwargs):
+            Counting.calls += 1
+            return super().get_key_cache(*args, **kwargs)
+
+    def run(cls, patch):
+        cache = cls(cfg, batch_size=1, max_length=2500, device=str(gpu), sparse_budget=1024, rank=64, max_decode_len=4)
+        synthesize_state(cache, 2500, seed=7, cos_sin=table)
+        attn = ShadowAttention(cache, 4, 128, 1024, lambda q, k, p: (q, k), None, table)
+        joined = attn._joined(cache)
+        if patch:
+            real = cache.get_key_cache
+            cache.get_key_cache = lambda *a, **k: (patch.append(1), real(*a, **k))[1]
+        q = torch.ones(1, 8, 1, 128, dtype=torch.bfloat16, device=gpu)
+        kv = torch.ones(1, 2, 1, 128, dtype=torch.bfloat16, device=gpu)
+        out = attn.decode(q, kv, kv, None, 0)
+        torch.cuda.synchronize()
+        return joined, out
+
+    joined, want = run(ShadowKVCache_CPU, None)
+    assert joined
+    joined, got = run(Counting, None)
+    assert not joined and Counting.calls == 1 and torch.equal(got, want)
+    hits = [0]
+    _, got = run(ShadowKVCache_CPU, hits)
+    assert len(hits) == 2 and torch.equal(got, want)
