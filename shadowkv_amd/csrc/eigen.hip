@@ -650,7 +650,8 @@ extern "C" int skv_sym_eig_top(const float* a, int batch, int n, int rank, float
                      reinterpret_cast<ulonglong2*>(ws + l.xchg), words, g.tickets, status, batch);
   auto run = [&](auto nrv) {
     constexpr int NR = decltype(nrv)::value;
-    hipLaunchKernelGGL(tridiag_kernel<NR>, dim3(256), dim3(kWgWaves * 64), 0, s, g);
+    // 64 workgroups per XCD where the dispatcher deals them round robin, at most 32 of them with a part.
+    hipLaunchKernelGGL(tridiag_kernel<NR>, dim3(512), dim3(kWgWaves * 64), 0, s, g);
     hipLaunchKernelGGL(bisect_kernel, dim3(rank, batch), dim3(kPoints), 0, s, g, 64 * NR);
     hipLaunchKernelGGL(backtransform_kernel<NR>, dim3(rank, batch), dim3(64), 0, s, g);
   };
