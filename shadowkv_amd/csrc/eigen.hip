@@ -24,6 +24,7 @@
 // MI355X, rank 160, us in all: n = 1024 2190 (the reduction 1640, 1.6 a step; the eigenpairs of T 360; the
 // back transformation 180), n = 512 848, n = 256 386 (1.0 a step: the exchange and the chain of
 // reductions alone); rocSOLVER's full decomposition 19600, 10400, 4900.
+#include <mutex>
 #include <type_traits>
 
 #include "wave_reduce.h"
@@ -248,13 +249,11 @@ struct Reduction {
 // (One wave per SIMD with up to 512 registers: 8 columns of 1024 rows are 128 of them; two waves of
 // 4 columns would do the redundant vector work twice.)
 // A workgroup takes its part by its order of arrival on its XCD: problem b runs on XCD b, its
-// 2 NR workgroups one per CU on an idle device (a
-// request for LDS that forces it changes nothing, and small workgroups let two calls run side by side).
+// 2 NR workgroups one per CU on an idle device (a request for LDS that forces it changes nothing).
 template <int NR>
 __global__ void __launch_bounds__(kWgWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 tridiag_kernel(EigenArgs g) {
   using Red = Reduction<NR>;
-  // Two of the buffers are used; the size keeps a second workgroup off the CU (160 KB of LDS).
   __shared__ float2 pc[2][Red::kPad];
   __shared__ int part;
   const int b = static_cast<int>(__builtin_amdgcn_s_getreg(kHwRegXccId) & 15u);
@@ -589,6 +588,17 @@ __global__ void __launch_bounds__(256) prepare_kernel(ulonglong2* xchg, int64_t 
   if (i < batch) status[i] = 0;
 }
 
+// Reductions of one device run one after another, whatever their streams: the 2 NR workgroups of a problem
+// wait for one another, an XCD holds 64 of them, and of three calls at n = 1024 each could hold a share and
+// wait until it gives up (three threads: 156 ms a round of calls, most without a result; in turn 5.2). Two beside each
+// other were no faster than in turn. A captured call is not ordered: its event would belong to the graph.
+struct ReductionOrder {
+  std::mutex mutex;
+  hipEvent_t done = nullptr;  // after the newest reduction
+  bool recorded = false;
+};
+ReductionOrder g_order[64];
+
 int blocks_of(int n) { return n <= 128 ? 2 : n <= 256 ? 4 : n <= 512 ? 8 : 16; }
 
 struct Layout {
@@ -648,16 +658,41 @@ extern "C" int skv_sym_eig_top(const float* a, int batch, int n, int rank, float
   const int64_t words = static_cast<int64_t>(batch) * n * 64 * nr / 2;
   hipLaunchKernelGGL(prepare_kernel, dim3(static_cast<unsigned>((words + 255) / 256)), dim3(256), 0, s,
                      reinterpret_cast<ulonglong2*>(ws + l.xchg), words, g.tickets, status, batch);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  int device = 0;
+  if (hipStreamIsCapturing(s, &capture) != hipSuccess || hipGetDevice(&device) != hipSuccess || device < 0 ||
+      device >= 64) {
+    skv_set_error("%s: no stream state or device", what);
+    return SKV_ELAUNCH;
+  }
+  const bool ordered = capture == hipStreamCaptureStatusNone;
+  ReductionOrder& order = g_order[device];
   auto run = [&](auto nrv) {
     constexpr int NR = decltype(nrv)::value;
+    std::unique_lock<std::mutex> lock(order.mutex, std::defer_lock);
+    if (ordered) {
+      lock.lock();
+      if (!order.done && hipEventCreateWithFlags(&order.done, hipEventDisableTiming) != hipSuccess) return false;
+      if (order.recorded && hipStreamWaitEvent(s, order.done, 0) != hipSuccess) return false;
+    }
     // 64 workgroups per XCD where the dispatcher deals them round robin, at most 32 of them with a part.
     hipLaunchKernelGGL(tridiag_kernel<NR>, dim3(512), dim3(kWgWaves * 64), 0, s, g);
+    if (ordered) {
+      if (hipEventRecord(order.done, s) != hipSuccess) return false;
+      order.recorded = true;
+      lock.unlock();
+    }
     hipLaunchKernelGGL(bisect_kernel, dim3(rank, batch), dim3(kPoints), 0, s, g, 64 * NR);
     hipLaunchKernelGGL(backtransform_kernel<NR>, dim3(rank, batch), dim3(64), 0, s, g);
+    return true;
   };
-  if (nr == 2) run(std::integral_constant<int, 2>{});
-  else if (nr == 4) run(std::integral_constant<int, 4>{});
-  else if (nr == 8) run(std::integral_constant<int, 8>{});
-  else run(std::integral_constant<int, 16>{});
+  const bool launched = nr == 2   ? run(std::integral_constant<int, 2>{})
+                        : nr == 4 ? run(std::integral_constant<int, 4>{})
+                        : nr == 8 ? run(std::integral_constant<int, 8>{})
+                                  : run(std::integral_constant<int, 16>{});
+  if (!launched) {
+    skv_set_error("%s: no event to order the reductions by", what);
+    return SKV_ELAUNCH;
+  }
   return skv_check_launch(what);
 }

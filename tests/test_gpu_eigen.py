@@ -1,5 +1,7 @@
 """The leading eigenpairs of symmetric positive semidefinite matrices (skv_sym_eig_top) against the
 float64 eigendecomposition, and the factors where the kernel's result is not taken."""
+import threading
+
 import pytest
 import torch
 
@@ -91,3 +93,33 @@ def test_batches_past_the_xcds(gpu):
     want = (uu[..., :20] * s[:, None, :20]) @ vh[:, :20]
     got = (u @ svt).cpu().double()
     assert ((got - want).norm(dim=(1, 2)) / want.norm(dim=(1, 2))).max() < 1e-3
+
+
+def test_concurrent_streams(gpu):
+    """Calls of several threads and streams, more than an XCD holds together (two at n = 1024), all give
+    the result of a call alone, to the bit."""
+    _say("eigen: four streams")
+    g = torch.Generator().manual_seed(2)
+    x = torch.randn(4, 1200, 1024, generator=g).to(gpu)
+    grams = [torch.matmul(k.T.contiguous(), k)[None].contiguous() for k in x]
+    want = [shadowkv.sym_eig_top(a, 16) for a in grams]
+    torch.cuda.synchronize()
+    got = [[] for _ in grams]
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(5):
+                got[i].append(shadowkv.sym_eig_top(grams[i], 16))
+        stream.synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i, (w, vt, _) in enumerate(want):
+        assert len(got[i]) == 5
+        for gw, gvt, status in got[i]:
+            assert status.tolist() == [1]
+            assert torch.equal(gw, w) and torch.equal(gvt, vt)
