@@ -59,6 +59,14 @@ def causal_attention_fp32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, blo
 JOINED_FETCH_WORKGROUPS = 128
 
 
+def _unreplaced(obj, steps: dict) -> bool:
+    """Whether obj's methods named in steps are the functions that steps holds: not another class's, not a
+    subclass's and not the instance's own."""
+    return all(getattr(type(obj), n, None) is f for n, f in steps.items()) and steps.keys().isdisjoint(vars(obj))
+
+
+# What prefill() runs in two halves where nobody has replaced it.
+_PREFILL_STEPS = {"prefill_kv_cache": ShadowKVCache_CPU.prefill_kv_cache}
 # The steps of decode_begin() that the joined chain of decode() does otherwise.
 _CACHE_STEPS = ("get_retrieval_position_ids", "get_value_cache", "get_key_cache", "move_value_hits")
 _ATTENTION_STEPS = ("decode_begin", "decode_begin_appended", "_key_path")
@@ -70,18 +78,17 @@ class ShadowAttention(AttentionBase):
         kv_cache = self.kv_cache
         kv_cache.get_svd(key_states, layer_idx=layer_idx)
         query_states, key_states = self.apply_rotary_pos_emb(query_states, key_states, position_ids)
-        # The values' copy to the host runs beside the attention, and the attention's launch comes before
-        # the state's many small ones, whose issue by the host it covers (MI355X, one layer: 8192
-        # tokens on 8 kv heads 4.17 -> 3.74 ms, 19333 on 2 7.14 -> 6.51 ms).
-        copy = kv_cache._value_copy = kv_cache.start_value_copy(value_states, layer_idx)
-        try:
-            out = causal_attention_fp32(query_states, key_states, value_states)
+        if not _unreplaced(kv_cache, _PREFILL_STEPS):  # (what it does with the values comes before the attention)
             kv_cache.prefill_kv_cache(value_states, layer_idx, key_states, query_states[:, :, -1:])
+            return causal_attention_fp32(query_states, key_states, value_states)
+        # prefill_kv_cache in its two halves: the values' copy to the host runs beside the attention, and the
+        # attention's launch comes before the state's many small ones, whose issue by the host it covers
+        # (MI355X, one layer: 8192 tokens on 8 kv heads 4.17 -> 3.74 ms, 19333 on 2 7.14 -> 6.51 ms).
+        pending = kv_cache._begin_prefill(value_states, layer_idx, key_states, query_states[:, :, -1:])
+        try:
+            return causal_attention_fp32(query_states, key_states, value_states)
         finally:
-            kv_cache._value_copy = None
-            if copy is not None:
-                copy.synchronize()
-        return out
+            kv_cache._end_prefill(pending)
 
     def decode(self, query_states, key_states, value_states, position_ids, layer_idx):
         """One new token through the layer: decode_begin() and decode_end(). Nothing can overlap the

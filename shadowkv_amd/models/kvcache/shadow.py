@@ -211,7 +211,6 @@ class ShadowKVCache_CPU(KVCacheBase):
         self.attn_workspace = None
         self.attn_out = None
         self.select_workspace = None  # allocated with the landmarks
-        self._value_copy = None  # a value copy started for the next prefill_kv_cache (its event)
         # Device-resident append row / attention length (use_device_lengths); None = host integers.
         self.append_row_dev = None
         self.kv_len_dev = None
@@ -335,10 +334,9 @@ class ShadowKVCache_CPU(KVCacheBase):
 
     def start_value_copy(self, new_v_cache: torch.Tensor, layer_idx: int):
         """Begins the copy of a prompt's value chunks to the layer's pinned host store on the fetch stream,
-        beside the work that follows on the current one. Returns the event that prefill_kv_cache waits for
-        on the host, or None where prefill_kv_cache makes the copy itself: a store in device memory, values
-        whose rows are not contiguous, tracing. A caller that starts the copy of a prompt's values early
-        leaves the event in _value_copy for the prefill_kv_cache call on the same values."""
+        beside the work that follows on the current one. Returns the event to wait for on the host (the
+        values unchanged and alive until then), or None where it does not apply and nothing was started: a
+        store in device memory, values whose rows are not contiguous, tracing."""
         bsz, H, incoming, D = new_v_cache.shape
         c, pb = self.chunk_size, self.prefilled_batch
         n = incoming // c
@@ -346,7 +344,7 @@ class ShadowKVCache_CPU(KVCacheBase):
         v = new_v_cache
         if not (self.value_store == "host" and plain_eager(v) and v.dtype == store.dtype and v.stride(-1) == 1
                 and v.stride(-2) == D and 0 < n <= store.shape[2] and pb + bsz <= store.shape[0] and bsz * H <= 64
-                and not torch.cuda.is_current_stream_capturing()):
+                and v.device == self.copy_stream.device and not torch.cuda.is_current_stream_capturing()):
             return None
         dst = store[pb:pb + bsz, :, :n]
         src = v[:, :, :n * c]
@@ -367,9 +365,16 @@ class ShadowKVCache_CPU(KVCacheBase):
         (skv_chunk_stats); the outlier chunks and the landmark ids (skv_select_outliers); the
         landmarks (skv_gather_rows); outlier and initially selected K/V chunks copied by the
         chunk-gather kernel; the initial selection by the decode path's scoring, GQA max and top-k."""
+        self._end_prefill(self._begin_prefill(new_v_cache, layer_idx, key_states_roped, last_query_states))
+
+    def _begin_prefill(self, new_v_cache: torch.Tensor, layer_idx: int, key_states_roped: torch.Tensor,
+                       last_query_states: torch.Tensor = None):
+        """First half of prefill_kv_cache: its checks, the geometry and the value chunks' way to the store,
+        which may still run when this returns, beside what the caller issues before _end_prefill() of the
+        result (always called, and the values left as they are until then)."""
         self._require_device(new_v_cache, key_states_roped, last_query_states)
         bsz, H, incoming, D = new_v_cache.shape
-        c, pb, l, G = self.chunk_size, self.prefilled_batch, layer_idx, self.num_key_value_groups
+        c, pb, l = self.chunk_size, self.prefilled_batch, layer_idx
         max_ctx_chunks = incoming // c
         if max_ctx_chunks > self.v_cache_cpu[l].shape[2]:
             raise ValueError(f"prompt of {incoming} tokens exceeds max_length {self.max_length}")
@@ -377,18 +382,21 @@ class ShadowKVCache_CPU(KVCacheBase):
         v = new_v_cache if new_v_cache.stride(-1) == 1 and new_v_cache.stride(-2) == D else new_v_cache.contiguous()
         k = key_states_roped if key_states_roped.stride(-1) == 1 and key_states_roped.stride(-2) == D \
             else key_states_roped.contiguous()
-        value_copy, self._value_copy = self._value_copy, None
-        if value_copy is None:
-            value_copy = self.start_value_copy(v, l)
+        value_copy = self.start_value_copy(v, l)
         if value_copy is None:
             self.v_cache_cpu[l][pb:pb + bsz, :, :max_ctx_chunks].copy_(
                 v[:, :, :self.max_ctx_chunks_len].reshape(bsz, H, max_ctx_chunks, c * D))
+        return k, v, l, last_query_states, value_copy
+
+    def _end_prefill(self, pending):
+        """Second half of prefill_kv_cache, on the stream _begin_prefill() ran on."""
+        k, v, l, last_query_states, value_copy = pending
         try:
             self._encode_layer(k, v, l, last_query_states)
         finally:
             if value_copy is not None:  # the host store is whole when this returns (and v may be freed)
                 value_copy.synchronize()
-        self._finish_layer(l, bsz, incoming)
+        self._finish_layer(l, v.shape[0], v.shape[2])
 
     def _encode_layer(self, k: torch.Tensor, v: torch.Tensor, l: int, last_query_states: torch.Tensor):
         """The device part of prefill_kv_cache: buffers, landmarks and the initial selection."""

@@ -129,3 +129,68 @@ def test_prefill_value_copy(gpu, ctx, max_length, B, first):
             assert torch.equal(got[lo:hi, :, :n], v[lo:hi, :, :n * c].reshape(hi - lo, H, n, c * D).cpu())
             assert not got[:, :, n:].any() and not got[hi:].any()
         del cache, attn
+
+
+def test_prefill_replaced_kv_cache_step(gpu, monkeypatch):
+    """A prefill_kv_cache replaced in a subclass, on the class, on the instance or in another cache
+    altogether: the store holds the values that it passed on, not those that prefill was given, and the
+    attention takes the values as it left them."""
+    from shadowkv_amd.models.attention import ShadowAttention, shadow
+    from shadowkv_amd.models.tensor_op import build_cos_sin_cache
+    _say("prefill with a replaced prefill_kv_cache")
+    H, G, D, ctx, c = 2, 2, 128, 1400, 8
+    cfg = types.SimpleNamespace(num_attention_heads=G * H, num_key_value_heads=H, hidden_size=G * H * D,
+                                num_hidden_layers=1)
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn(1, h, ctx, D, generator=g).to(torch.bfloat16).to(gpu) for h in (G * H, H, H))
+    table = build_cos_sin_cache(ctx, 10000.0, D, device=gpu)
+    make = dict(batch_size=1, max_length=ctx, device=str(gpu), sparse_budget=1024, rank=32)
+    real = ShadowKVCache_CPU.prefill_kv_cache
+
+    def scaled(self, values, *args):
+        real(self, 2 * values, *args)
+
+    def in_place(self, values, *args):
+        real(self, values.mul_(2), *args)
+
+    class Delegating:  # the methods that prefill calls, and no others
+        def __init__(self, inner):
+            self.get_svd, self.prefill_kv_cache = inner.get_svd, inner.prefill_kv_cache
+
+    for form in ("subclass", "class", "instance", "in place", "delegating", "none"):
+        factor = 1 if form in ("delegating", "none") else 2
+        with monkeypatch.context() as m:
+            cls = ShadowKVCache_CPU
+            if form in ("subclass", "in place"):
+                cls = type("Replacing", (cls,), {"prefill_kv_cache": scaled if form == "subclass" else in_place})
+            cache = cls(cfg, **make)
+            if form == "class":
+                m.setattr(ShadowKVCache_CPU, "prefill_kv_cache", scaled)
+            if form == "instance":
+                cache.prefill_kv_cache = types.MethodType(scaled, cache)
+            attn = ShadowAttention(Delegating(cache) if form == "delegating" else cache, G, D, G * H * D,
+                                   lambda a, b, p: (a, b), None, table)
+            given = v.clone()
+            out = attn.prefill(q, k, given, None, 0)
+            want = (factor * v).view(1, H, ctx // c, c * D).cpu()
+            assert torch.equal(cache.v_cache_cpu[0][:, :, :ctx // c], want), form
+            used = 2 * v if form == "in place" else v
+            assert torch.equal(given, used) and torch.equal(out, shadow.causal_attention_fp32(q, k, used)), form
+
+
+def test_prefill_refusals_leave_the_store(gpu):
+    """A prompt that prefill_kv_cache refuses leaves the store as it was, through prefill too."""
+    from shadowkv_amd.models.attention import ShadowAttention
+    from shadowkv_amd.models.tensor_op import build_cos_sin_cache
+    _say("refused prompts")
+    H, G, D, ctx = 2, 2, 128, 1400
+    cfg = types.SimpleNamespace(num_attention_heads=G * H, num_key_value_heads=H, hidden_size=G * H * D,
+                                num_hidden_layers=1)
+    q, k, v = (torch.ones(1, h, ctx, D, dtype=torch.bfloat16, device=gpu) for h in (G * H, H, H))
+    cache = ShadowKVCache_CPU(cfg, batch_size=1, max_length=ctx, device=str(gpu), sparse_budget=1024, rank=32)
+    attn = ShadowAttention(cache, G, D, G * H * D, lambda a, b, p: (a, b.cpu()), None,
+                           build_cos_sin_cache(ctx, 10000.0, D, device=gpu))
+    with pytest.raises(ValueError, match="device"):  # keys on the host
+        attn.prefill(q, k, v, None, 0)
+    torch.cuda.synchronize()
+    assert not cache.v_cache_cpu[0].any() and cache.prefilled_batch == 0
