@@ -429,7 +429,7 @@ int skv_keys_factors(const uint16_t* keys, int64_t stride_b, int64_t stride_h, i
  * G = q_heads / kv_heads, 128-element bf16 rows with unit element stride, fp32 scores, probabilities
  * and sums, one rounding to bf16. q, k, v: 16-byte aligned rows (strides multiples of 8 elements; a
  * stride may be 0), out 8-byte. workspace: skv_prefill_attn_workspace_bytes bytes, 16-byte aligned
- * (the transposed values), overwritten. */
+ * (the transposed values and a flag per 64 keys), overwritten. */
 int64_t skv_prefill_attn_workspace_bytes(int batch_size, int kv_heads, int len);
 int skv_prefill_attn(const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_s, const uint16_t* k,
                      int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_s, const uint16_t* v,

@@ -11,17 +11,21 @@
 //
 // Probabilities keep their fp32 value: p is cut by truncation into three bf16 parts (8 + 8 + 8
 // significant bits, an exact sum) and P.V is three MFMAs into one fp32 accumulator, so nothing is
-// rounded to 16 bits before the output. The maximum that the exponentials are taken against is only
+// rounded to 16 bits before the output. A part may be zero, and its product with an infinite value
+// NaN, where the whole p gives the infinity: where the keys' values hold an infinity or a NaN (vt_kernel
+// says so per tile) the second and third products take them as zeros. The maximum that the exponentials are taken against is only
 // moved when a score passes it by 2^8 (the ratio of the sums does not depend on it), which leaves
 // the 64 accumulators of a lane alone in most tiles.
 //
 // A workgroup of 4 waves owns 128 queries of one head (32 per wave) and walks the keys in tiles of
-// 64 (two workgroups per CU: 64 KB of LDS, 195 VGPRs), K and V^T tiles double-buffered in LDS by direct global-to-LDS loads (K's 16-byte chunks
+// 64 (two workgroups per CU: 64 KB of LDS, 209 VGPRs), K and V^T tiles double-buffered in LDS by direct global-to-LDS loads (K's 16-byte chunks
 // swizzled by the row at the source, so that operand reads have no bank conflicts).
 //
 // MI355X, 32 query heads: 8 kv heads x 8192 tokens 0.93 ms (591 TFLOP/s of the causal 4 L^2 D / 2 count,
 // 1180 with the three-part P.V that is issued: the rate of a large bf16 GEMM here is 1120) against
 // 11.5 ms for fp32 torch operations over 1024-query blocks; 2 kv heads x 19333 tokens 4.8 ms against 58.
+#include <type_traits>
+
 #include "skv_common.h"
 
 namespace {
@@ -40,19 +44,26 @@ constexpr int kTile16 = kTileKeys * kD * 2 / 16;  // 16-byte chunks of a K or V^
 constexpr int kXcds = 8;
 
 // vt[row][key / 16][dim][16 keys], the keys of a group of 16 in the order 0-3, 8-11, 4-7, 12-15; zeros past L.
+// odd[row][key / 64]: whether the tile holds an infinity or a NaN.
 __global__ void __launch_bounds__(256) vt_kernel(const uint16_t* __restrict__ v, int64_t sb, int64_t sh, int64_t ss,
-                                                 int H, int L, u32x4* __restrict__ vt, int groups) {
+                                                 int H, int L, u32x4* __restrict__ vt, int groups,
+                                                 int* __restrict__ odd) {
   __shared__ uint16_t t[64][kD + 2];
   const int row = blockIdx.y, b = row / H, h = row - b * H;
   const int k0 = blockIdx.x * 64;
   const uint16_t* src = v + b * sb + h * sh;
+  bool not_finite = false;
   for (int i = threadIdx.x; i < 64 * 16; i += 256) {
     const int r = i >> 4, c = i & 15;
     const u32x4 x = skv::load16_or_zero(src + static_cast<int64_t>(min(k0 + r, L - 1)) * ss + 8 * c, k0 + r < L);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) *reinterpret_cast<uint32_t*>(&t[r][8 * c + 2 * e]) = x[e];
+    for (int e = 0; e < 4; ++e) {
+      *reinterpret_cast<uint32_t*>(&t[r][8 * c + 2 * e]) = x[e];
+      not_finite |= (x[e] & 0x7f80u) == 0x7f80u || (x[e] & 0x7f800000u) == 0x7f800000u;
+    }
   }
-  __syncthreads();
+  not_finite = __syncthreads_or(not_finite);
+  if (threadIdx.x == 0) odd[row * gridDim.x + blockIdx.x] = not_finite;
   // 16-byte chunk i: group i / 256, dim (i % 256) / 2, half i % 2
   for (int i = threadIdx.x; i < 4 * 256; i += 256) {
     const int g = i >> 8, d = (i >> 1) & 127, hf = i & 1;
@@ -72,6 +83,7 @@ struct PrefillArgs {
   const uint16_t* k;
   int64_t k_sb, k_sh, k_ss;
   const u32x4* vt;
+  const int* odd;
   uint16_t* out;
   int64_t o_sb, o_sh, o_ss;
   int Hq, Hkv, G, L, qblocks, rows;  // rows = B * Hkv
@@ -82,6 +94,16 @@ struct PrefillArgs {
 __device__ __forceinline__ void load_lds(const void* src, u32x4* dst) {
   __builtin_amdgcn_global_load_lds(
       (const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+// Infinities and NaNs of bf16 pairs as zeros.
+__device__ __forceinline__ u32x4 finite_part(u32x4 x) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if ((x[e] & 0x7f80u) == 0x7f80u) x[e] &= 0xffff0000u;
+    if ((x[e] & 0x7f800000u) == 0x7f800000u) x[e] &= 0x0000ffffu;
+  }
+  return x;
 }
 
 __device__ __forceinline__ float other_half_max(float x) {
@@ -124,10 +146,11 @@ __global__ void __launch_bounds__(kWaves * 64, 2) prefill_attn_kernel(PrefillArg
   const int query = q0 + li;
 
   const uint16_t* kbase = a.k + b * a.k_sb + h * a.k_sh;
-  const u32x4* vbase = a.vt + static_cast<int64_t>(bh) * ((a.L + kTileKeys - 1) / kTileKeys) * kTile16;
+  const int row_tiles = (a.L + kTileKeys - 1) / kTileKeys;
+  const u32x4* vbase = a.vt + static_cast<int64_t>(bh) * row_tiles * kTile16;
   const int tiles = (min(a.L, qb * kQBlock + kQBlock) + kTileKeys - 1) / kTileKeys;
   const int krow = wave * 16 + (lane >> 4);  // + 4 i: this lane's K rows of a tile
-  auto issue = [&](int t, u32x4* kd, u32x4* vd) {
+  auto issue = [&](int t, u32x4* kd, u32x4* vd) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = krow + 4 * i;
@@ -153,7 +176,7 @@ __global__ void __launch_bounds__(kWaves * 64, 2) prefill_attn_kernel(PrefillArg
   float m = -INFINITY;  // the reference the exponentials are taken against, in units of log2
   float l = 0.f;        // this lane's share of the row sum
 
-  auto compute = [&](int t, const u32x4* kt, const u32x4* vt) {
+  auto compute = [&](auto special, int t, const u32x4* kt, const u32x4* vt) __attribute__((always_inline)) {
     const int k0 = t * kTileKeys;
     if (k0 > q0 + kQWave - 1) return;  // wave-uniform: all keys after the wave's last query
     f32x16 s[2];
@@ -217,27 +240,37 @@ __global__ void __launch_bounds__(kWaves * 64, 2) prefill_attn_kernel(PrefillArg
 #pragma unroll
       for (int d = 0; d < 4; ++d) vf[d] = vt[gk * 256 + (32 * d + li) * 2 + half];
 #pragma unroll
-      for (int i = 0; i < 3; ++i)
+      for (int i = 0; i < 3; ++i) {
+        if (decltype(special)::value && i == 1)
+#pragma unroll
+          for (int d = 0; d < 4; ++d) vf[d] = finite_part(vf[d]);
 #pragma unroll
         for (int d = 0; d < 4; ++d)
           o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[d]),
                                                          __builtin_bit_cast(bf16x8, p[i]), o[d], 0, 0, 0);
+      }
     }
   };
 
-  issue(0, ka, va);
-  for (int t = 0; t < tiles; t += 2) {
-    // Tile t is in ka / va (every wave has waited for its own loads into LDS, which __syncthreads
-    // alone does not do), and every wave is past tile t - 1 in kb / vb.
-    skv::drain_and_barrier();
-    if (t + 1 < tiles) issue(t + 1, kb, vb);
-    compute(t, ka, va);
-    if (t + 1 < tiles) {
+  auto walk = [&](auto special) __attribute__((always_inline)) {
+    for (int t = 0; t < tiles; t += 2) {
+      // Tile t is in ka / va (every wave has waited for its own loads into LDS, which __syncthreads
+      // alone does not do), and every wave is past tile t - 1 in kb / vb.
       skv::drain_and_barrier();
-      if (t + 2 < tiles) issue(t + 2, ka, va);
-      compute(t + 1, kb, vb);
+      if (t + 1 < tiles) issue(t + 1, kb, vb);
+      compute(special, t, ka, va);
+      if (t + 1 < tiles) {
+        skv::drain_and_barrier();
+        if (t + 2 < tiles) issue(t + 2, ka, va);
+        compute(special, t + 1, kb, vb);
+      }
     }
-  }
+  };
+  issue(0, ka, va);
+  bool odd = false;
+  for (int t = threadIdx.x; t < tiles; t += kWaves * 64) odd |= a.odd[bh * row_tiles + t] != 0;
+  if (__syncthreads_or(odd)) walk(std::true_type{});  // workgroup-uniform
+  else walk(std::false_type{});
 
   if (query < a.L) {
     const auto ls = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
@@ -259,7 +292,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 extern "C" int64_t skv_prefill_attn_workspace_bytes(int batch_size, int kv_heads, int len) {
   if (batch_size < 1 || kv_heads < 1 || len < 1) return 0;
-  return static_cast<int64_t>(batch_size) * kv_heads * ((len + kTileKeys - 1) / kTileKeys) * kTile16 * 16;
+  return static_cast<int64_t>(batch_size) * kv_heads * ((len + kTileKeys - 1) / kTileKeys) * (kTile16 * 16 + 4);
 }
 
 extern "C" int skv_prefill_attn(const uint16_t* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_s,
@@ -301,9 +334,10 @@ extern "C" int skv_prefill_attn(const uint16_t* q, int64_t q_stride_b, int64_t q
   }
   const hipStream_t s = static_cast<hipStream_t>(stream);
   u32x4* vt = static_cast<u32x4*>(workspace);
+  int* odd = reinterpret_cast<int*>(vt + rows * tiles * kTile16);
   hipLaunchKernelGGL(vt_kernel, dim3(tiles, static_cast<unsigned>(rows)), dim3(256), 0, s, v, v_stride_b, v_stride_h,
-                     v_stride_s, kv_heads, len, vt, tiles * 4);
-  PrefillArgs a{q, q_stride_b, q_stride_h, q_stride_s, k, k_stride_b, k_stride_h, k_stride_s, vt, out,
+                     v_stride_s, kv_heads, len, vt, tiles * 4, odd);
+  PrefillArgs a{q, q_stride_b, q_stride_h, q_stride_s, k, k_stride_b, k_stride_h, k_stride_s, vt, odd, out,
                 o_stride_b, o_stride_h, o_stride_s, q_heads, kv_heads, G, len, qblocks, static_cast<int>(rows),
                 scale * 1.44269504088896340736f};
   hipLaunchKernelGGL(prefill_attn_kernel, dim3(static_cast<unsigned>(grid)), dim3(kWaves * 64), 0, s, a);

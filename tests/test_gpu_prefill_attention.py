@@ -87,3 +87,32 @@ def test_differentiated_and_other_calls_stay_with_torch(gpu):
         dq = torch.autograd.forward_ad.make_dual(q, torch.ones_like(q))
         out = torch.autograd.forward_ad.unpack_dual(shadow.causal_attention_fp32(dq, k, v))
         assert out.tangent is not None
+
+
+@pytest.mark.parametrize("L,at", [(1, 0), (70, 0), (200, 3), (200, 64), (300, 130)])
+def test_prefill_attn_infinite_values(gpu, L, at):
+    """An infinite value reaches every query that sees its key, whatever the bits of its probability (the
+    first query's is exactly 1), of either sign; both signs of one dim, and a NaN, give NaN. The other
+    dims and the queries of earlier tiles (64 keys) are as without."""
+    _say(f"prefill_attn infinite values L={L} at={at}")
+    g = torch.Generator().manual_seed(L + at)
+    q, k, v = (torch.randn(1, h, L, 128, generator=g).to(torch.bfloat16) for h in (4, 2, 2))
+    q[:, :, : L // 2] = 0.0  # equal scores: probabilities 1 / (i + 1), half of them short in binary
+    plain = shadowkv.prefill_attn(q.to(gpu), k.to(gpu), v.to(gpu)).cpu()
+    inf = float("inf")
+    v[0, 0, at, 5], v[0, 0, at, 6], v[0, 1, at, 7], v[0, 1, L - 1, 7], v[0, 1, at, 9] = inf, -inf, inf, -inf, float("nan")
+    out = shadowkv.prefill_attn(q.to(gpu), k.to(gpu), v.to(gpu)).cpu()
+    seen = out[0, at:]  # [queries, heads, dims]: heads 0, 1 read kv head 0 and heads 2, 3 kv head 1
+    last = max(0, (L - 1) // 64 * 64 - at)  # from this one on a query's own tile holds the last key's -inf
+    assert (seen[:, :2, 5] == inf).all() and (seen[:, :2, 6] == -inf).all()
+    if at == L - 1:
+        assert (seen[:, 2:, 7] == -inf).all()  # (the same key: overwritten)
+    else:
+        assert (seen[:last, 2:, 7] == inf).all() and seen[-1, 2:, 7].isnan().all()
+    assert seen[:, 2:, 9].isnan().all()
+    same = torch.ones(4, 128, dtype=torch.bool)
+    same[:2, 5:7] = False
+    same[2:, [7, 9]] = False
+    assert torch.equal(out[0][:, same], plain[0][:, same])
+    first = min(at, L - 1) // 64 * 64
+    assert torch.equal(out[0, :first], plain[0, :first])
