@@ -67,9 +67,11 @@ def _unreplaced(obj, steps: dict) -> bool:
 
 # What prefill() runs in two halves where nobody has replaced it.
 _PREFILL_STEPS = {"prefill_kv_cache": ShadowKVCache_CPU.prefill_kv_cache}
-# The steps of decode_begin() that the joined chain of decode() does otherwise.
-_CACHE_STEPS = ("get_retrieval_position_ids", "get_value_cache", "get_key_cache", "move_value_hits")
-_ATTENTION_STEPS = ("decode_begin", "decode_begin_appended", "_key_path")
+# The steps of decode_begin() that the joined chain of decode() does otherwise, and those that it takes in
+# their place.
+_CACHE_STEPS = {n: getattr(ShadowKVCache_CPU, n) for n in (
+    "get_retrieval_position_ids", "get_value_cache", "get_key_cache", "move_value_hits", "one_stream_active",
+    "fetch_and_rebuild")}
 
 
 class ShadowAttention(AttentionBase):
@@ -109,18 +111,10 @@ class ShadowAttention(AttentionBase):
         return self.decode_end((query_states, key_states, value_states, [], layer_idx))
 
     def _joined(self, kv_cache) -> bool:
-        """Whether decode() may take the joined chain: a cache in its default setting, and neither class's
-        steps of the two-stream chain replaced (they would not be called)."""
-        if kv_cache.pooled or kv_cache.fold_hit_moves or getattr(kv_cache, "key_stream", None) is not None:
-            return False
-        cache_type, own = type(kv_cache), vars(kv_cache)
-        if cache_type is not ShadowKVCache_CPU and any(
-                getattr(cache_type, n) is not getattr(ShadowKVCache_CPU, n) for n in _CACHE_STEPS):
-            return False
-        if type(self) is not ShadowAttention and any(
-                getattr(type(self), n) is not getattr(ShadowAttention, n) for n in _ATTENTION_STEPS):
-            return False
-        return not any(n in own for n in _CACHE_STEPS) and not any(n in vars(self) for n in _ATTENTION_STEPS)
+        """Whether decode() may take the joined chain: a ShadowKVCache_CPU in its default setting, and no step
+        of either chain replaced, in the cache or here (it would not be called, or not as it expects)."""
+        return (_unreplaced(kv_cache, _CACHE_STEPS) and _unreplaced(self, _ATTENTION_STEPS) and not kv_cache.pooled
+                and not kv_cache.fold_hit_moves and kv_cache.key_stream is None)
 
     def decode_begin(self, query_states, key_states, value_states, position_ids, layer_idx):
         """First half of decode(): RoPE, append, chunk selection, the value fetch launched on the
@@ -195,3 +189,6 @@ class ShadowAttention(AttentionBase):
                                     kv_len_dev=kv_cache.kv_len_dev, pool=pool,
                                     vstore=kv_cache.value_store_args(layer_idx))
         return out.view(B, 1, Hq, -1)
+
+
+_ATTENTION_STEPS = {n: getattr(ShadowAttention, n) for n in ("decode_begin", "decode_begin_appended", "_key_path")}

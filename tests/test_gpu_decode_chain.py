@@ -103,3 +103,47 @@ def test_replaced_steps_are_called(gpu):
     hits = [0]
     _, got = run(ShadowKVCache_CPU, hits)
     assert len(hits) == 2 and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("form", ["class", "delegating", "fetch_and_rebuild", "attention class"])
+def test_other_replacements_keep_the_chain(gpu, form, monkeypatch):
+    """A step patched on the class itself, a cache of another class that hands its attributes on, a
+    fetch_and_rebuild with the arguments it had, and an attention step patched on the class."""
+    _say(f"decode chain: {form}")
+    cfg = types.SimpleNamespace(num_attention_heads=8, num_key_value_heads=2, hidden_size=1024, num_hidden_layers=1)
+    table = build_cos_sin_cache(3000, 500000.0, 128, device=gpu)
+    calls = []
+
+    class Own(ShadowKVCache_CPU):
+        def fetch_and_rebuild(self, layer_idx, position_ids, cos_sin_cache):
+            raise AssertionError("not a step of the two-stream chain")
+
+    class Delegating:
+        def __init__(self, inner):
+            self._inner = inner
+
+        def __getattr__(self, name):
+            return getattr(self._inner, name)
+
+    def run(patched):
+        cls = Own if patched and form == "fetch_and_rebuild" else ShadowKVCache_CPU
+        cache = cls(cfg, batch_size=1, max_length=2500, device=str(gpu), sparse_budget=1024, rank=64, max_decode_len=4)
+        synthesize_state(cache, 2500, seed=7, cos_sin=table)
+        if patched and form == "delegating":
+            cache = Delegating(cache)
+        attn = ShadowAttention(cache, 4, 128, 1024, lambda q, k, p: (q, k), None, table)
+        assert attn._joined(cache) != patched
+        q = torch.ones(1, 8, 1, 128, dtype=torch.bfloat16, device=gpu)
+        kv = torch.ones(1, 2, 1, 128, dtype=torch.bfloat16, device=gpu)
+        out = attn.decode(q, kv, kv, None, 0)
+        torch.cuda.synchronize()
+        return out
+
+    want = run(False)
+    if form in ("class", "attention class"):
+        owner, name = {"class": (ShadowKVCache_CPU, "get_key_cache"),
+                       "attention class": (ShadowAttention, "_key_path")}[form]
+        real = getattr(owner, name)
+        monkeypatch.setattr(owner, name, lambda self, *a, **k: (calls.append(1), real(self, *a, **k))[1])
+    assert torch.equal(run(True), want)
+    assert len(calls) == (form in ("class", "attention class"))
