@@ -264,7 +264,8 @@ int skv_select_chunks_ws(const uint16_t* D, const float* norm, const float* sum,
  * into its last launch: after the reorder, the workgroup that owns row r compacts the row's hits
  * in place in each non-null buffer, exactly as skv_gather_copy_d2d_with_offsets would with the
  * offsets and cnts just written: slot(i) <- slot(offsets[r,i]) for i < cnts[r], where
- *   slot(i) = buffer + r*buf_stride + buf_offset + i*chunk_elems   (bf16 elements).
+ *   slot(i) = buffer + r*buf_stride + buf_offset + i*chunk_elems   (bf16 elements)
+ * (as launches that follow where LDS holds the chunk bitmaps but no slot list beside them).
  * Requires position_ids/offsets/cnts (the reorder), chunk_elems a positive multiple of 8,
  * buf_offset and buf_stride multiples of 8, buf_stride >= buf_offset + select_sets*chunk_elems and
  * 16-byte aligned buffers. With it the value buffer needs only the host-link half of the fetch

@@ -951,8 +951,11 @@ int select_impl(const char* what, const uint16_t* D, const float* norm, const fl
   while (P < select_sets) P <<= 1;
   const int words = reorder ? (num_chunks + 31) / 32 : 0;
   const size_t base_lds = (static_cast<size_t>(words) * 8 + static_cast<size_t>(P) * 8 + 15) / 16 * 16;
-  // the hits' old slots, for the folded hit moves
-  const size_t fixed = base_lds + (move ? (static_cast<size_t>(select_sets) * 4 + 15) / 16 * 16 : 0);
+  // The hits' old slots, for the folded hit moves; where they do not fit beside the bitmaps any more (the last
+  // 1.4% of the chunk counts that do), the moves are launches of their own after the selection.
+  const size_t hit_lds = move ? (static_cast<size_t>(select_sets) * 4 + 15) / 16 * 16 : 0;
+  const bool fold = move && base_lds + hit_lds <= kLdsBudget;
+  const size_t fixed = base_lds + (fold ? hit_lds : 0);
   if (fixed > kLdsBudget) {
     skv_set_error("%s: %d chunks need %zu bytes of bitmap, above the LDS budget", what, num_chunks, fixed);
     return SKV_EUNSUPPORTED;
@@ -979,7 +982,7 @@ int select_impl(const char* what, const uint16_t* D, const float* norm, const fl
   a.vec = (n % 8 == 0 && (reinterpret_cast<uintptr_t>(D) & 15u) == 0 &&
            (!out_scores || (reinterpret_cast<uintptr_t>(out_scores) & 15u) == 0));
   a.keys_off = static_cast<int>(fixed);
-  a.hit_src_off = move ? static_cast<int>(base_lds) : 0;
+  a.hit_src_off = fold ? static_cast<int>(base_lds) : 0;
   a.mv_buf[0] = mv_v;
   a.mv_buf[1] = mv_k;
   a.mv_offset = mv_offset;
@@ -1032,6 +1035,14 @@ int select_impl(const char* what, const uint16_t* D, const float* norm, const fl
                       : skv_softmax_gqa_max(D, norm, sum, nullptr, out_scores, rows, m, n, stream);
     if (rc) return rc;
   }
+  auto finish = [&]() -> int {
+    int rc = skv_check_launch(what);
+    for (uint16_t* buf : {mv_v, mv_k})
+      if (!rc && buf && !fold)
+        rc = skv_gather_copy_d2d_with_offsets(buf, offsets, cnts, rows, 1, static_cast<int64_t>(select_sets) * mv_chunk,
+                                              mv_offset, mv_stride, select_sets, mv_chunk, stream);
+    return rc;
+  };
   if (parts) {
     PartArgs pa{};
     pa.scores = out_scores;
@@ -1050,13 +1061,13 @@ int select_impl(const char* what, const uint16_t* D, const float* norm, const fl
     hipLaunchKernelGGL(part_emit_kernel, pg, dim3(kPartThreads), 0, st, pa);
     const size_t fb = (fixed + 15) / 16 * 16;
     hipLaunchKernelGGL(select_finish_kernel, dim3(rows), dim3(kThreads), fb, st, a, pa);
-    return skv_check_launch(what);
+    return finish();
   }
   // (keys precomputed: the query count plays no part, and the MP = 4 instance keeps them in registers)
   if (m <= 4 || split) hipLaunchKernelGGL(select_kernel<4>, dim3(rows), dim3(kThreads), ldsb, st, a);
   else if (m <= 8) hipLaunchKernelGGL(select_kernel<8>, dim3(rows), dim3(kThreads), ldsb, st, a);
   else hipLaunchKernelGGL(select_kernel<16>, dim3(rows), dim3(kThreads), ldsb, st, a);
-  return skv_check_launch(what);
+  return finish();
 }
 
 }  // namespace

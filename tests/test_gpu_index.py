@@ -446,3 +446,52 @@ def test_select_chunks_folded_hit_moves(gpu, monkeypatch, rows, m, n, S, chunk_e
         assert (cnts == expect).all()
     if mode == "shift" and S >= 4:
         assert (cnts >= 2 * (S // 4)).all() and (offs[:, S // 4] == S // 4 + 1).all()
+
+
+@pytest.mark.parametrize("split", ["0", "1", "ws"])
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+def test_select_chunks_hit_moves_at_the_bitmaps_limit(gpu, monkeypatch, extra, split):
+    """Chunk counts whose bitmaps fill the selection's LDS (150 KB): the largest that leaves room for the folded
+    moves' slot list (extra 0), one bitmap word past it and one below. All are served, as by the plain
+    selection and the separate moves, and one word past the largest count of that is refused by both."""
+    monkeypatch.setenv("SKV_SELECT_SPLIT", {"ws": "2"}.get(split, split))
+    rows, m, n, S, chunk_elems = 2, 4, 600, 512, 64
+    budget, keys = 150 * 1024, 512 * 8
+    nchunks = ((budget - keys - 4 * S) // 16 * 2 + extra) * 32
+    _say(f"select_chunks moves at the LDS limit chunks={nchunks} split={split}")
+    g = torch.Generator().manual_seed(5)
+    q = torch.randn(rows, m, 128, generator=g).to(torch.bfloat16).to(gpu)
+    L = torch.randn(rows, n, 128, generator=g).to(torch.bfloat16).to(gpu)
+    lidx = torch.stack([torch.randperm(nchunks, generator=g)[:n].sort().values for _ in range(rows)]).to(gpu)
+    lidx[:, -1] = nchunks - 1
+    tiles = (n + 255) // 256
+    D = torch.empty(rows, m, n, dtype=torch.bfloat16, device=gpu)
+    norm = torch.empty(rows, m, tiles, device=gpu)
+    ssum = torch.empty_like(norm)
+    shadowkv.score_logits(q, L, D, norm, ssum, rows, m, n, 128)
+    ws = torch.empty(shadowkv.select_workspace_bytes(rows, n, S), dtype=torch.uint8, device=gpu) if split == "ws" else None
+    old = torch.stack([lidx[r, torch.randperm(n, generator=g)[:S].to(gpu)] for r in range(rows)])
+    stride = S * chunk_elems
+    bufs = [torch.randn(rows, stride, generator=g).to(torch.bfloat16).to(gpu) for _ in range(2)]
+
+    def select(chunks, move):
+        pos, off = old.clone(), torch.empty(rows * S, dtype=torch.int32, device=gpu)
+        cnt = torch.empty(rows, dtype=torch.int32, device=gpu)
+        shadowkv.select_chunks(D, norm, ssum, rows, m, n, lidx, S, chunks, pos, off, cnt, workspace=ws, move=move,
+                               out_scores=torch.empty(rows, n, dtype=torch.bfloat16, device=gpu))
+        torch.cuda.synchronize()
+        return pos, off, cnt
+
+    pos, off, cnt = select(nchunks, None)
+    want = [b.clone() for b in bufs]
+    for b in want:
+        shadowkv.gather_copy_d2d_with_offsets(b, off, cnt, 1, rows, S * chunk_elems, 0, stride, S)
+    assert 0 < int(cnt.min()) and int(cnt.max()) < S
+    got = [b.clone() for b in bufs]
+    again = select(nchunks, (got[0], got[1], 0, stride, chunk_elems))
+    assert all(torch.equal(a, b) for a, b in zip(again, (pos, off, cnt)))
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    past = ((budget - keys) // 16 * 2 + 1) * 32
+    for move in (None, (bufs[0], bufs[1], 0, stride, chunk_elems)):
+        with pytest.raises(RuntimeError, match="LDS"):
+            select(past, move)
