@@ -147,3 +147,34 @@ def test_other_replacements_keep_the_chain(gpu, form, monkeypatch):
         monkeypatch.setattr(owner, name, lambda self, *a, **k: (calls.append(1), real(self, *a, **k))[1])
     assert torch.equal(run(True), want)
     assert len(calls) == (form in ("class", "attention class"))
+
+
+def _fetch_launches(gpu, monkeypatch, **attrs):
+    """The fetch workgroups that decode() asks for, of a cache with the given settings."""
+    from shadowkv_amd.kernels import shadowkv
+    cfg = types.SimpleNamespace(num_attention_heads=8, num_key_value_heads=2, hidden_size=1024, num_hidden_layers=1)
+    table = build_cos_sin_cache(3000, 500000.0, 128, device=gpu)
+    cache = ShadowKVCache_CPU(cfg, batch_size=1, max_length=2500, device=str(gpu), sparse_budget=1024, rank=64,
+                              max_decode_len=4, value_store=attrs.pop("value_store", "host"))
+    for name, value in attrs.items():
+        setattr(cache, name, value)
+    synthesize_state(cache, 2500, seed=7, cos_sin=table)
+    attn = ShadowAttention(cache, 4, 128, 1024, lambda q, k, p: (q, k), None, table)
+    real, asked = shadowkv.fetch_misses_rebuild_k_rope, []
+    with monkeypatch.context() as m:
+        m.setattr(shadowkv, "fetch_misses_rebuild_k_rope",
+                  lambda *a, fetch_workgroups=0, **k: (asked.append(fetch_workgroups),
+                                                       real(*a, fetch_workgroups=fetch_workgroups, **k))[1])
+        q = torch.ones(1, 8, 1, 128, dtype=torch.bfloat16, device=gpu)
+        kv = torch.ones(1, 2, 1, 128, dtype=torch.bfloat16, device=gpu)
+        attn.decode(q, kv, kv, None, 0)
+        torch.cuda.synchronize()
+    return asked
+
+
+def test_fetch_workgroups_of_a_gathered_device_store(gpu, monkeypatch):
+    """A store in device memory that is gathered from: the library's own count for it, or the cache's."""
+    _say("decode chain: fetch workgroups of a device store")
+    assert _fetch_launches(gpu, monkeypatch, value_store="device", values_in_place=False) == [0]
+    assert _fetch_launches(gpu, monkeypatch, value_store="device", values_in_place=False,
+                           fused_fetch_workgroups=40) == [40]
