@@ -21,13 +21,15 @@ constexpr int kChunksPerFetchWG = 16;  // miss chunks per fetch tile
 // fastest GLM-4-9B one (418.5 vs 414.0 / 415.3 / 407.4 at 32 / 96 / 160).
 constexpr int kDefaultFetchWGs = 48;
 
+inline int env_workgroups(const char* name) {  // 0: not set, or out of range
+  const char* e = getenv(name);
+  const int v = e ? atoi(e) : 0;
+  return (v >= 1 && v <= 65536) ? v : 0;
+}
+
 inline int fetch_workgroups() {
-  static const int wgs = [] {
-    const char* e = getenv("SKV_FETCH_WGS");
-    const int v = e ? atoi(e) : 0;
-    return (v >= 1 && v <= 65536) ? v : kDefaultFetchWGs;
-  }();
-  return wgs;
+  static const int env = env_workgroups("SKV_FETCH_WGS");
+  return env ? env : kDefaultFetchWGs;
 }
 
 // Fetch workgroups (of 4 waves' worth) of a launch that also rebuilds keys (fetch_rebuild_kernel,
@@ -39,12 +41,20 @@ inline int fetch_workgroups() {
 constexpr int kDefaultFusedFetchWGs = 64;
 
 inline int fused_fetch_workgroups_target() {
-  static const int wgs = [] {
-    const char* e = getenv("SKV_FUSED_FETCH_WGS");
-    const int v = e ? atoi(e) : 0;
-    return (v >= 1 && v <= 65536) ? v : kDefaultFusedFetchWGs;
-  }();
-  return wgs;
+  static const int env = env_workgroups("SKV_FUSED_FETCH_WGS");
+  return env ? env : kDefaultFusedFetchWGs;
+}
+
+// The same for a launch that no other work runs beside (a decode() call), from a store in host memory: with
+// nothing but the rebuild to slow down, which the host reads do little to, more of them in flight win (us per
+// call at 64 / 96 / 128 / 256: 4 x 122880 tokens, 2048 selected, 258 / 246 / 242 / 243; 3 x 28426, 4096
+// selected, 292 / 259 / 250 / 256; 4 x 50000, 1024 selected in chunks of 4, 157 / 154 / 152 / 154). Both environment
+// variables override it, the launch's own before the one of the value fetch that it stands in for.
+constexpr int kAloneFetchWGs = 128;
+
+inline int fetch_workgroups_alone() {
+  static const int fused = env_workgroups("SKV_FUSED_FETCH_WGS"), fetch = env_workgroups("SKV_FETCH_WGS");
+  return fused ? fused : fetch ? fetch : kAloneFetchWGs;
 }
 
 // Whether the value store at p is device memory (a store kept in HBM, e.g. value_store="device"

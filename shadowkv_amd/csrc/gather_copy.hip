@@ -131,6 +131,8 @@ int check_common(const char* what, const void* a, const void* b, int batch_size,
 
 }  // namespace
 
+extern "C" int skv_fetch_workgroups_alone(void) { return skv::fetch_workgroups_alone(); }
+
 extern "C" int skv_gather_copy_d2d_with_offsets(void* keys, const int32_t* offsets, const int32_t* cnts,
                                                 int batch_size, int heads, int64_t gpu_k_length,
                                                 int64_t gpu_k_offset, int64_t gpu_k_stride, int map_size,

@@ -17,6 +17,7 @@ sparse_attn_decode) expose the fused kernels used by the decode path.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -394,6 +395,13 @@ def _rebuild_geometry(u, sv, position_ids, cnts, cos_sin, cache, sparse_start, c
         raise ValueError("position_ids must be contiguous along the chunk axis")
     _need(cnts, B * H, "cnts")
     return u_sb, u_sh, u_sr, u_rows, sv_sb, sv_sh, sv_sn, mode, rank
+
+
+@functools.lru_cache(maxsize=None)
+def fetch_workgroups_alone() -> int:
+    """The fetch workgroups of a fetch_misses_rebuild_k_rope launch from pinned host memory that no other work
+    runs beside: the library's count, or SKV_FUSED_FETCH_WGS or SKV_FETCH_WGS of the environment (read once)."""
+    return _lib.lib().skv_fetch_workgroups_alone()
 
 
 def fetch_misses_rebuild_k_rope(values, v_cache_buffer, offsets, cnts, cpu_v_length, gpu_v_offset, gpu_v_stride,

@@ -51,15 +51,6 @@ def causal_attention_fp32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, blo
     return out
 
 
-# Fetch workgroups of a decode() call: with nothing beside the launch but the rebuild, which the host reads
-# slow, more of them in flight win over the default of 64 for a store in host memory, which suits lanes whose fetches run
-# beside dense layers (MI355X, us per call at 64 / 96 / 128 / 256: 4 x 122880 tokens, 2048 selected, 258 / 246 /
-# 242 / 243; 3 x 28426, 4096 selected, 292 / 259 / 250 / 256; 4 x 50000, 1024 selected in chunks of 4, 157 / 154 /
-# 152 / 154). A store in device memory that is gathered from keeps the library's default for it (512; 16 x 60000,
-# 2048 selected, us at 64 / 128 / 512: 271 / 214 / 201).
-JOINED_FETCH_WORKGROUPS = 128
-
-
 def _unreplaced(obj, steps: dict) -> bool:
     """Whether obj's methods named in steps are the functions that steps holds: not another class's, not a
     subclass's and not the instance's own."""
@@ -107,8 +98,8 @@ class ShadowAttention(AttentionBase):
         kv_cache.update_kv_cache(key_states, value_states, layer_idx)
         position_ids = kv_cache.get_retrieval_position_ids(layer_idx=layer_idx, query_states=query_states, fold_all=True)
         workgroups = kv_cache.fused_fetch_workgroups
-        if not workgroups and kv_cache.value_store == "host":
-            workgroups = JOINED_FETCH_WORKGROUPS
+        if not workgroups and kv_cache.value_store == "host":  # (the default for device memory suits this too)
+            workgroups = shadowkv.fetch_workgroups_alone()
         key_states, value_states = kv_cache.fetch_and_rebuild(layer_idx, position_ids, self.cos_sin_cache,
                                                               fetch_workgroups=workgroups)
         return self.decode_end((query_states, key_states, value_states, [], layer_idx))

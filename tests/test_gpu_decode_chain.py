@@ -178,3 +178,13 @@ def test_fetch_workgroups_of_a_gathered_device_store(gpu, monkeypatch):
     assert _fetch_launches(gpu, monkeypatch, value_store="device", values_in_place=False) == [0]
     assert _fetch_launches(gpu, monkeypatch, value_store="device", values_in_place=False,
                            fused_fetch_workgroups=40) == [40]
+
+
+def test_fetch_workgroups_of_a_host_store(gpu, monkeypatch):
+    """A store in host memory: the library's count for a launch alone (which the environment overrides), or the
+    cache's."""
+    from shadowkv_amd.kernels import shadowkv
+    _say("decode chain: fetch workgroups of a host store")
+    monkeypatch.setattr(shadowkv, "fetch_workgroups_alone", lambda *a: 33)
+    assert _fetch_launches(gpu, monkeypatch) == [33]
+    assert _fetch_launches(gpu, monkeypatch, fused_fetch_workgroups=40) == [40]

@@ -1,5 +1,10 @@
 """The C-ABI library loads on a CPU-only host and exports every function the header declares."""
 import ctypes
+import os
+import subprocess
+import sys
+
+import pytest
 
 from shadowkv_amd import _lib
 
@@ -117,3 +122,14 @@ def test_build_rejects_kernels_that_use_scratch():
         "x.hip:9:1: remark:     ScratchSize [bytes/lane]: 320 [-Rpass-analysis=kernel-resource-usage]",
     ])
     assert build.scratch_kernels(remarks) == [("k_spills", 320)]
+
+
+@pytest.mark.parametrize("env,want", [({}, 128), ({"SKV_FETCH_WGS": "40"}, 40), ({"SKV_FUSED_FETCH_WGS": "72"}, 72),
+                                      ({"SKV_FETCH_WGS": "40", "SKV_FUSED_FETCH_WGS": "72"}, 72),
+                                      ({"SKV_FETCH_WGS": "0"}, 128)])
+def test_fetch_workgroups_follow_the_environment(env, want):
+    """The fetch workgroups of a decode() call: the documented variables, read once per process."""
+    code = f"import ctypes; print(ctypes.CDLL({str(_lib.LIB_PATH)!r}).skv_fetch_workgroups_alone())"
+    clean = {k: v for k, v in os.environ.items() if k not in ("SKV_FETCH_WGS", "SKV_FUSED_FETCH_WGS")}
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100, env={**clean, **env})
+    assert r.returncode == 0 and int(r.stdout) == want, (r.stdout, r.stderr)
