@@ -57,6 +57,15 @@ def _unreplaced(obj, steps: dict) -> bool:
     return all(getattr(type(obj), n, None) is f for n, f in steps.items()) and steps.keys().isdisjoint(vars(obj))
 
 
+# Selected tokens (sparse_budget) up to which the joined chain is taken, by value store: its selection moves a row's
+# hits with the row's one workgroup, and a wide selection's moves then take longer than the compaction
+# launches over the whole device, which a host store's fetch overlaps besides (MI355X, us per call, two-stream /
+# joined, batch 1, 2, 4 of 120000 tokens and 8 kv heads; host, 8192 selected: 254 / 250, 393 / 384, 660 / 655; 16384:
+# 375 / 402, 599 / 630, 1051 / 1112; device, 16384: 173 / 142, 173 / 168, 217 / 222, gathered from 213 / 212; 32768:
+# 189 / 210, 231 / 258, 370 / 402).
+JOINED_MAX_BUDGET = {"host": 8192, "device": 16384}
+
+
 # What prefill() runs in two halves where nobody has replaced it.
 _PREFILL_STEPS = {"prefill_kv_cache": ShadowKVCache_CPU.prefill_kv_cache}
 # The steps of decode_begin() that the joined chain of decode() does otherwise, and those that it takes in
@@ -105,10 +114,12 @@ class ShadowAttention(AttentionBase):
         return self.decode_end((query_states, key_states, value_states, [], layer_idx))
 
     def _joined(self, kv_cache) -> bool:
-        """Whether decode() may take the joined chain: a ShadowKVCache_CPU in its default setting, and no step
-        of either chain replaced, in the cache or here (it would not be called, or not as it expects)."""
+        """Whether decode() takes the joined chain: a ShadowKVCache_CPU in its default setting, no step of either
+        chain replaced, in the cache or here (it would not be called, or not as it expects), and a selection
+        that it is the faster one for (JOINED_MAX_BUDGET)."""
         return (_unreplaced(kv_cache, _CACHE_STEPS) and _unreplaced(self, _ATTENTION_STEPS) and not kv_cache.pooled
-                and not kv_cache.fold_hit_moves and kv_cache.key_stream is None)
+                and not kv_cache.fold_hit_moves and kv_cache.key_stream is None
+                and kv_cache.sparse_budget <= JOINED_MAX_BUDGET[kv_cache.value_store])
 
     def decode_begin(self, query_states, key_states, value_states, position_ids, layer_idx):
         """First half of decode(): RoPE, append, chunk selection, the value fetch launched on the

@@ -188,3 +188,32 @@ def test_fetch_workgroups_of_a_host_store(gpu, monkeypatch):
     monkeypatch.setattr(shadowkv, "fetch_workgroups_alone", lambda *a: 33)
     assert _fetch_launches(gpu, monkeypatch) == [33]
     assert _fetch_launches(gpu, monkeypatch, fused_fetch_workgroups=40) == [40]
+
+
+@pytest.mark.parametrize("store,budget,joined", [("host", 8192, True), ("host", 16384, False), ("device", 16384, True),
+                                                 ("device", 32768, False)])
+def test_wide_selections_keep_the_two_streams(gpu, monkeypatch, store, budget, joined):
+    """A selection too wide for its rows' workgroups to move the hits: the two-stream chain, with the bits of
+    the joined one."""
+    _say(f"decode chain {store} budget={budget}")
+    from shadowkv_amd.models.attention import shadow
+    ctx, chunk = 60000, 16
+    cfg = types.SimpleNamespace(num_attention_heads=8, num_key_value_heads=2, hidden_size=1024, num_hidden_layers=1)
+    table = build_cos_sin_cache(ctx + 8, 500000.0, 128, device=gpu)
+    g = torch.Generator(device=gpu).manual_seed(1)
+    base = torch.randn(1, 8, 1, 128, generator=g, device=gpu)
+    qs = [(0.95 * base + 0.3 * torch.randn(1, 8, 1, 128, generator=g, device=gpu)).to(torch.bfloat16) for _ in range(3)]
+    kv = torch.randn(1, 2, 1, 128, generator=g, device=gpu).to(torch.bfloat16)
+    got = []
+    for force in (False, True):
+        cache = ShadowKVCache_CPU(cfg, batch_size=1, max_length=ctx, device=str(gpu), sparse_budget=budget,
+                                  chunk_size=chunk, rank=64, max_decode_len=4, value_store=store)
+        synthesize_state(cache, ctx, seed=7, cos_sin=table)
+        attn = ShadowAttention(cache, 4, 128, 1024, lambda q, k, p: (q, k), None, table)
+        if force:
+            monkeypatch.setitem(shadow.JOINED_MAX_BUDGET, store, budget if not joined else budget - 1)
+        assert attn._joined(cache) == (joined != force)
+        got.append([attn.decode(q, kv, kv, None, 0) for q in qs] + [cache.position_ids, cache.cnts])
+        torch.cuda.synchronize()
+    assert int(got[0][-1].max()) > 0
+    assert all(torch.equal(a, b) for a, b in zip(*got))
