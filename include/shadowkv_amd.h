@@ -465,9 +465,10 @@ int skv_fetch_misses_rebuild_k_rope(const void* values, void* v_cache_buffer, co
                                     int rank, int head_dim, int fetch_workgroups, int rebuild_workgroups,
                                     void* stream);
 
-/* The fetch_workgroups for such a launch from pinned host memory that no other work runs beside: the
- * library's count (128), or SKV_FUSED_FETCH_WGS, else SKV_FETCH_WGS, of the environment (read once). */
-int skv_fetch_workgroups_alone(void);
+/* The fetch_workgroups for such a launch from pinned host memory that no other work runs beside, for rows
+ * rows of num_chunks slots: the library's count (128, or 384 past 768 tiles of 16 slots), or SKV_FUSED_FETCH_WGS,
+ * else SKV_FETCH_WGS, of the environment (read once). */
+int skv_fetch_workgroups_alone(int rows, int num_chunks);
 
 /* ---- f3: device chunk pool (a GPU cache of P >= S chunk slots per (b, h) and layer) ------
  * No reference counterpart: extends the slot reuse of reorder_keys_and_compute_offsets

@@ -29,7 +29,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "skv_gather_copy_misses_with_offsets": (_i32, [_p, _p, _p, _p, _i32, _i32, _i64, _i64, _i64, _i64, _i32, _i32,
                                                     _p]),
     "skv_gather_copy_d2d_with_offsets": (_i32, [_p, _p, _p, _i32, _i32, _i64, _i64, _i64, _i32, _i32, _p]),
-    "skv_fetch_workgroups_alone": (_i32, []),
+    "skv_fetch_workgroups_alone": (_i32, [_i32, _i32]),
     "skv_gather_copy": (_i32, [_p, _p, _p, _i32, _i32, _i64, _i64, _i32, _i32, _p]),
     "skv_apply_rotary_pos_emb_new": (
         _i32, [_p, _p, _p, _p, _i32, _i32, _i32, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i32, _i64,

@@ -46,15 +46,17 @@ inline int fused_fetch_workgroups_target() {
 }
 
 // The same for a launch that no other work runs beside (a decode() call), from a store in host memory: with
-// nothing but the rebuild to slow down, which the host reads do little to, more of them in flight win (us per
-// call at 64 / 96 / 128 / 256: 4 x 122880 tokens, 2048 selected, 258 / 246 / 242 / 243; 3 x 28426, 4096
-// selected, 292 / 259 / 250 / 256; 4 x 50000, 1024 selected in chunks of 4, 157 / 154 / 152 / 154). Both environment
-// variables override it, the launch's own before the one of the value fetch that it stands in for.
-constexpr int kAloneFetchWGs = 128;
+// nothing but the rebuild to slow down, which the host reads do little to, more of them in flight win, and
+// past 768 tiles the more so (us per call at 64 / 128 / 384; 3 x 28426 tokens, 4096 selected (768 tiles) 294 / 252 /
+// 252; 4 x 122880, 2048 (512) 263 / 242 / 243; 4 x 50000, 1024 in chunks of 4 (512) 157 / 153 / 155; 8 x 60000, 2048
+// (1024) 378 / 382 / 373; 12 x 60000, 2048 (1536) 551 / 538 / 523; 16 x 60000, 2048 (2048) 679 / 689 / 676; 24 x 30011,
+// 2048 (3072) 869 / 907 / 873). Both environment variables override it, the launch's own before the one of the
+// value fetch that it stands in for.
+constexpr int kAloneFetchWGs = 128, kAloneFetchWGsMany = 384, kAloneFewTiles = 768;
 
-inline int fetch_workgroups_alone() {
+inline int fetch_workgroups_alone(int tiles) {
   static const int fused = env_workgroups("SKV_FUSED_FETCH_WGS"), fetch = env_workgroups("SKV_FETCH_WGS");
-  return fused ? fused : fetch ? fetch : kAloneFetchWGs;
+  return fused ? fused : fetch ? fetch : tiles <= kAloneFewTiles ? kAloneFetchWGs : kAloneFetchWGsMany;
 }
 
 // Whether the value store at p is device memory (a store kept in HBM, e.g. value_store="device"

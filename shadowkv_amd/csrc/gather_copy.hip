@@ -131,7 +131,11 @@ int check_common(const char* what, const void* a, const void* b, int batch_size,
 
 }  // namespace
 
-extern "C" int skv_fetch_workgroups_alone(void) { return skv::fetch_workgroups_alone(); }
+extern "C" int skv_fetch_workgroups_alone(int rows, int num_chunks) {
+  if (rows < 1 || num_chunks < 1) return 0;
+  const int64_t tiles = static_cast<int64_t>(rows) * ((num_chunks + skv::kChunksPerFetchWG - 1) / skv::kChunksPerFetchWG);
+  return skv::fetch_workgroups_alone(static_cast<int>(std::min<int64_t>(tiles, INT32_MAX)));
+}
 
 extern "C" int skv_gather_copy_d2d_with_offsets(void* keys, const int32_t* offsets, const int32_t* cnts,
                                                 int batch_size, int heads, int64_t gpu_k_length,

@@ -17,7 +17,6 @@ sparse_attn_decode) expose the fused kernels used by the decode path.
 from __future__ import annotations
 
 import ctypes
-import functools
 import math
 
 import torch
@@ -397,11 +396,11 @@ def _rebuild_geometry(u, sv, position_ids, cnts, cos_sin, cache, sparse_start, c
     return u_sb, u_sh, u_sr, u_rows, sv_sb, sv_sh, sv_sn, mode, rank
 
 
-@functools.lru_cache(maxsize=None)
-def fetch_workgroups_alone() -> int:
+def fetch_workgroups_alone(rows: int, num_chunks: int) -> int:
     """The fetch workgroups of a fetch_misses_rebuild_k_rope launch from pinned host memory that no other work
-    runs beside: the library's count, or SKV_FUSED_FETCH_WGS or SKV_FETCH_WGS of the environment (read once)."""
-    return _lib.lib().skv_fetch_workgroups_alone()
+    runs beside, for rows rows of num_chunks slots: the library's count, or SKV_FUSED_FETCH_WGS or
+    SKV_FETCH_WGS of the environment (read once)."""
+    return _lib.lib().skv_fetch_workgroups_alone(rows, num_chunks)
 
 
 def fetch_misses_rebuild_k_rope(values, v_cache_buffer, offsets, cnts, cpu_v_length, gpu_v_offset, gpu_v_stride,

@@ -57,9 +57,10 @@ def _unreplaced(obj, steps: dict) -> bool:
     return all(getattr(type(obj), n, None) is f for n, f in steps.items()) and steps.keys().isdisjoint(vars(obj))
 
 
-# Selected tokens (sparse_budget) up to which the joined chain is taken, by value store: its selection moves a row's
-# hits with the row's one workgroup, and a wide selection's moves then take longer than the compaction
-# launches over the whole device, which a host store's fetch overlaps besides (MI355X, us per call, two-stream /
+# Selected tokens (sparse_budget) up to which the joined chain is taken, by value store: its selection moves both
+# buffers' hits before the fetch can start, a row's with one workgroup, where the two-stream chain moves the
+# keys' beside a host store's fetch, and its moves keep four loads in flight a thread against the compaction
+# kernel's eight (MI355X, us per call, two-stream /
 # joined, batch 1, 2, 4 of 120000 tokens and 8 kv heads; host, 8192 selected: 254 / 250, 393 / 384, 660 / 655; 16384:
 # 375 / 402, 599 / 630, 1051 / 1112; device, 16384: 173 / 142, 173 / 168, 217 / 222, gathered from 213 / 212; 32768:
 # 189 / 210, 231 / 258, 370 / 402).
@@ -108,7 +109,7 @@ class ShadowAttention(AttentionBase):
         position_ids = kv_cache.get_retrieval_position_ids(layer_idx=layer_idx, query_states=query_states, fold_all=True)
         workgroups = kv_cache.fused_fetch_workgroups
         if not workgroups and kv_cache.value_store == "host":  # (the default for device memory suits this too)
-            workgroups = shadowkv.fetch_workgroups_alone()
+            workgroups = shadowkv.fetch_workgroups_alone(kv_cache.block_num, kv_cache.select_sets)
         key_states, value_states = kv_cache.fetch_and_rebuild(layer_idx, position_ids, self.cos_sin_cache,
                                                               fetch_workgroups=workgroups)
         return self.decode_end((query_states, key_states, value_states, [], layer_idx))

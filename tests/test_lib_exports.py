@@ -124,12 +124,15 @@ def test_build_rejects_kernels_that_use_scratch():
     assert build.scratch_kernels(remarks) == [("k_spills", 320)]
 
 
-@pytest.mark.parametrize("env,want", [({}, 128), ({"SKV_FETCH_WGS": "40"}, 40), ({"SKV_FUSED_FETCH_WGS": "72"}, 72),
-                                      ({"SKV_FETCH_WGS": "40", "SKV_FUSED_FETCH_WGS": "72"}, 72),
-                                      ({"SKV_FETCH_WGS": "0"}, 128)])
+@pytest.mark.parametrize("env,want", [({}, "128 128 384 384"), ({"SKV_FETCH_WGS": "40"}, "40 40 40 40"),
+                                      ({"SKV_FUSED_FETCH_WGS": "72"}, "72 72 72 72"),
+                                      ({"SKV_FETCH_WGS": "40", "SKV_FUSED_FETCH_WGS": "72"}, "72 72 72 72"),
+                                      ({"SKV_FETCH_WGS": "0"}, "128 128 384 384")])
 def test_fetch_workgroups_follow_the_environment(env, want):
-    """The fetch workgroups of a decode() call: the documented variables, read once per process."""
-    code = f"import ctypes; print(ctypes.CDLL({str(_lib.LIB_PATH)!r}).skv_fetch_workgroups_alone())"
+    """The fetch workgroups of a decode() call by its tiles (16, 768, 769, past 2^31): the documented variables,
+    read once per process."""
+    code = (f"import ctypes; f = ctypes.CDLL({str(_lib.LIB_PATH)!r}).skv_fetch_workgroups_alone; "
+            "print(f(1, 256), f(48, 256), f(769, 16), f(2 ** 30, 2048))")
     clean = {k: v for k, v in os.environ.items() if k not in ("SKV_FETCH_WGS", "SKV_FUSED_FETCH_WGS")}
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100, env={**clean, **env})
-    assert r.returncode == 0 and int(r.stdout) == want, (r.stdout, r.stderr)
+    assert r.returncode == 0 and r.stdout.strip() == want, (r.stdout, r.stderr)
