@@ -399,7 +399,10 @@ int skv_gather_rows(const uint16_t* src, int rows, int src_rows, const int64_t* 
  * w [batch, rank] eigenvalues, descending; vt [batch, rank, n] their orthonormal eigenvectors, rows;
  * status [batch] 1 where the problem was solved. A status other than 1 leaves w and vt undefined: a
  * largest diagonal entry that is zero, not finite or beyond 2^+-100, or workgroups that did not come to run
- * beside one another in time (every wait is bounded). Eigenvalues closer than about 1e-9 of the largest
+ * beside one another in time (every wait is bounded). Calls of one process and device run their reductions in
+ * turn, whatever their streams; a call captured into a graph cannot be ordered, so its replays must not run
+ * beside another call or replay on the device (each could hold a share of the CUs that both wait for, until
+ * the waits run out). Eigenvalues closer than about 1e-9 of the largest
  * may have eigenvectors that are not orthogonal; callers check. batch <= 8 (one problem per XCD),
  * 2 <= n <= 1024, 1 <= rank <= n. workspace: skv_sym_eig_workspace_bytes bytes, 16-byte aligned. */
 int64_t skv_sym_eig_workspace_bytes(int batch, int n, int rank);

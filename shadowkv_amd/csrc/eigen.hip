@@ -656,8 +656,6 @@ extern "C" int skv_sym_eig_top(const float* a, int batch, int n, int rank, float
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int nr = blocks_of(n);
   const int64_t words = static_cast<int64_t>(batch) * n * 64 * nr / 2;
-  hipLaunchKernelGGL(prepare_kernel, dim3(static_cast<unsigned>((words + 255) / 256)), dim3(256), 0, s,
-                     reinterpret_cast<ulonglong2*>(ws + l.xchg), words, g.tickets, status, batch);
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   int device = 0;
   if (hipStreamIsCapturing(s, &capture) != hipSuccess || hipGetDevice(&device) != hipSuccess || device < 0 ||
@@ -665,6 +663,8 @@ extern "C" int skv_sym_eig_top(const float* a, int batch, int n, int rank, float
     skv_set_error("%s: no stream state or device", what);
     return SKV_ELAUNCH;
   }
+  hipLaunchKernelGGL(prepare_kernel, dim3(static_cast<unsigned>((words + 255) / 256)), dim3(256), 0, s,
+                     reinterpret_cast<ulonglong2*>(ws + l.xchg), words, g.tickets, status, batch);
   const bool ordered = capture == hipStreamCaptureStatusNone;
   ReductionOrder& order = g_order[device];
   auto run = [&](auto nrv) {

@@ -1078,7 +1078,9 @@ SYM_EIG_MAX_BATCH = 8
 def sym_eig_top(a, rank):
     """The `rank` leading eigenpairs of symmetric positive semidefinite a [b, n, n] (fp32, contiguous,
     b <= 8, 2 <= n <= 1024): (w [b, rank] descending, vt [b, rank, n], status [b] int32). Only rows of
-    status 1 hold a result, whose orthogonality within clusters of eigenvalues is the caller's to check."""
+    status 1 hold a result, whose orthogonality within clusters of eigenvalues is the caller's to check.
+    Captured into a graph, it must not be replayed beside another call or replay on the device: those run
+    in turn otherwise, and side by side they may run out of time (status 2 or 3)."""
     _dev(a, "a", torch.float32)
     if a.dim() != 3 or a.shape[1] != a.shape[2] or not a.is_contiguous():
         raise ValueError(f"sym_eig_top: a {tuple(a.shape)} must be contiguous [b, n, n]")

@@ -7,6 +7,7 @@ import torch
 
 from shadowkv_amd.kernels import shadowkv
 from shadowkv_amd.models.kvcache import shadow as kv
+from shadowkv_amd.streams import capture_graph
 
 pytestmark = pytest.mark.gpu
 
@@ -123,3 +124,24 @@ def test_concurrent_streams(gpu):
         for gw, gvt, status in got[i]:
             assert status.tolist() == [1]
             assert torch.equal(gw, w) and torch.equal(gvt, vt)
+
+
+def test_captured_call(gpu):
+    """Replays of a captured call, one after another with eager calls between them, give the eager result."""
+    _say("eigen: captured")
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(2, 700, 256, generator=g).to(gpu)
+    a = torch.matmul(x.transpose(1, 2).contiguous(), x)
+    want = shadowkv.sym_eig_top(a, 20)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with capture_graph(graph, gpu):
+        got = shadowkv.sym_eig_top(a, 20)
+    for _ in range(3):
+        for t in got:
+            t.fill_(7)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(u, v) for u, v in zip(got, want))
+        assert all(torch.equal(u, v) for u, v in zip(shadowkv.sym_eig_top(a, 20), want))
+        torch.cuda.synchronize()
