@@ -1075,6 +1075,13 @@ SYM_EIG_MAX_N = 1024
 SYM_EIG_MAX_BATCH = 8
 
 
+def sym_eig_runs_on(device) -> bool:
+    """Whether sym_eig_top's problems find the XCDs that they run on: a whole MI355X (8 XCDs of 32 CUs). In a
+    partition of one, XCDs are missing, and which ids the others have is not stated: problems of an absent id
+    would never be solved (their status stays 0), and every caller would pay for the attempt."""
+    return torch.cuda.get_device_properties(device).multi_processor_count >= 8 * 32
+
+
 def sym_eig_top(a, rank):
     """The `rank` leading eigenpairs of symmetric positive semidefinite a [b, n, n] (fp32, contiguous,
     b <= 8, 2 <= n <= 1024): (w [b, rank] descending, vt [b, rank, n], status [b] int32). Only rows of

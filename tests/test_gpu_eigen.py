@@ -1,6 +1,7 @@
 """The leading eigenpairs of symmetric positive semidefinite matrices (skv_sym_eig_top) against the
 float64 eigendecomposition, and the factors where the kernel's result is not taken."""
 import threading
+import types
 
 import pytest
 import torch
@@ -145,3 +146,20 @@ def test_captured_call(gpu):
         assert all(torch.equal(u, v) for u, v in zip(got, want))
         assert all(torch.equal(u, v) for u, v in zip(shadowkv.sym_eig_top(a, 20), want))
         torch.cuda.synchronize()
+
+
+def test_part_of_a_device_takes_eigh(gpu, monkeypatch):
+    """A device that reports fewer CUs than the XCDs of a whole one have: no attempt, eigh's factors."""
+    _say("eigen: part of a device")
+    g = torch.Generator().manual_seed(4)
+    k = torch.randn(1, 300, 128, generator=g).to(gpu)
+    u, svt = kv.low_rank_factors(k, 8)
+    monkeypatch.setattr(torch.cuda, "get_device_properties", lambda d: types.SimpleNamespace(multi_processor_count=128))
+    monkeypatch.setattr(shadowkv, "sym_eig_top", lambda *a: pytest.fail("attempted"))
+    assert kv._top_eigenpairs(torch.matmul(k.transpose(1, 2).contiguous(), k), 8) is None
+    cfg = types.SimpleNamespace(num_attention_heads=2, num_key_value_heads=1, hidden_size=256, num_hidden_layers=1)
+    cache = kv.ShadowKVCache_CPU(cfg, batch_size=1, max_length=300, device=str(gpu), sparse_budget=64, rank=8)
+    cache.U = torch.empty(1, device=gpu)
+    assert cache._keys_in_place(k.to(torch.bfloat16)) is None  # (their Gram matrix is not made for nothing)
+    u2, svt2 = kv.low_rank_factors(k, 8)
+    assert ((u2 @ svt2) - (u @ svt)).norm() <= 1e-4 * (u @ svt).norm()
