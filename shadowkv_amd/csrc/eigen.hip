@@ -35,7 +35,10 @@ constexpr int kCols = 8;        // columns per wave
 constexpr int kWgWaves = 4;     // waves per workgroup
 constexpr int kXccIds = 8;
 constexpr int kHwRegXccId = (3 << 11) | (0 << 6) | 20;  // s_getreg_b32 hwreg(HW_REG_XCC_ID, 0, 4)
-constexpr int kPollLimit = 1 << 19;                     // polls of one wait (a poll is ~0.5 us)
+// Polls of one wait, 28 ms at 0.22 us: longer than workgroups of other kernels keep this one's off the CUs, and not much
+// more than the full decomposition costs that the caller takes then. Three processes whose reductions meet on one
+// device (n = 1024; two fit beside one another) paid 114 ms a call at four times as many, 3.4 to 4.9 (one in ten 33) now.
+constexpr int kPollLimit = 1 << 17;
 constexpr int kMaxN = 1024;
 
 struct EigenArgs {
