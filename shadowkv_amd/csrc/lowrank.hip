@@ -19,10 +19,11 @@
 // project_kernel: a workgroup of 4 waves owns 256 rows and NT * 32 vectors, both operands by direct
 // loads into LDS (swizzled at the source), double-buffered in blocks of 32 columns.
 //
-// MI355X, 122880 x 1024 keys, rank 160: Gram matrix 385 us (671 TFLOP/s; conversion and fp32 product 2480),
+// MI355X, 122880 x 1024 keys, rank 160 (rank 64, 128, 192: factors 59, 114, 150): Gram matrix 385 us (671 TFLOP/s; conversion and fp32 product 2480),
 // factors 156 us (774 TFLOP/s issued; product, division, roundings and transposed copies 450); 3001 rows: 47
 // and 27 us against 70 and 43. Error of G against fp64 8e-8 (fp32 product: 5e-6); of U the same.
 #include <algorithm>
+#include <cstdint>
 #include <type_traits>
 
 #include "skv_common.h"
@@ -321,6 +322,41 @@ bool shape_ok(const char* what, const uint16_t* keys, int64_t sb, int64_t sh, in
   return true;
 }
 
+// Forms of project_kernel: a workgroup of `tiles` vector tiles (of 32) reads its rows of the keys once for all of
+// them, but is more work for one CU; 256 of them are a round of `us` at 1024 columns (further rounds take as long to
+// within a fifth), and the form whose rounds take least in all is taken. Measured with 1 / 2 / 3 / 4 / 5 / 6 tiles, us:
+// 122880 rows, rank 128 196 / 119 / 154 / 127, rank 160 242 / 163 / 154 / 214 / 141, rank 192 288 / 170 / 161 / 220 / 252 / 165;
+// 50000 rows, rank 128 75 / 52 / 67 / 59; 32768 rows, rank 160 52 / 49 / 47 / 55 / 64; 8192 rows, rank 160
+// 22 / 28 / 43 / 52 / 62: 4 and 6 tiles gain nowhere.
+struct ProjectForm {
+  int tiles, us;
+};
+constexpr ProjectForm kProjectForms[] = {{1, 19}, {2, 27}, {3, 40}, {5, 66}};
+
+int project_tiles(int rtiles, int64_t row_blocks) {
+  // (Three one-tile workgroups fit on a CU, so two rounds of them are little more than one: 19333 rows, rank 160
+  // 30 us against 35 with two tiles.)
+  if (row_blocks * rtiles <= 2 * 256) return 1;
+  int best = 1;
+  int64_t least = INT64_MAX;
+  for (const ProjectForm& f : kProjectForms) {
+    const int64_t us = (row_blocks * ((rtiles + f.tiles - 1) / f.tiles) + 255) / 256 * f.us;
+    if (f.tiles <= rtiles && us < least) {
+      least = us;
+      best = f.tiles;
+    }
+  }
+  return best;
+}
+
+// Rows of a part of v3: whole groups of any form.
+int padded_rank(int rank) {
+  const int rtiles = (rank + 31) / 32;
+  int most = 0;
+  for (const ProjectForm& f : kProjectForms) most = std::max(most, (rtiles + f.tiles - 1) / f.tiles * f.tiles);
+  return 32 * most;
+}
+
 }  // namespace
 
 extern "C" int64_t skv_keys_gram_workspace_bytes(int batch, int rows, int heads) {
@@ -358,7 +394,7 @@ extern "C" int skv_keys_gram(const uint16_t* keys, int64_t stride_b, int64_t str
 
 extern "C" int64_t skv_keys_factors_workspace_bytes(int batch, int heads, int rank) {
   if (batch < 1 || heads < 1 || heads * kD > kMaxN || rank < 1) return 0;
-  return static_cast<int64_t>(batch) * 3 * ((rank + 31) / 32 * 32) * heads * kD * 2;
+  return static_cast<int64_t>(batch) * 3 * padded_rank(rank) * heads * kD * 2;
 }
 
 extern "C" int skv_keys_factors(const uint16_t* keys, int64_t stride_b, int64_t stride_h, int64_t stride_s, int batch,
@@ -382,18 +418,21 @@ extern "C" int skv_keys_factors(const uint16_t* keys, int64_t stride_b, int64_t 
                   (long long)workspace_bytes, (long long)skv_keys_factors_workspace_bytes(batch, heads, rank));
     return SKV_EINVAL;
   }
-  const int rtiles = (rank + 31) / 32, rpad = 32 * rtiles;
+  const int rtiles = (rank + 31) / 32, rpad = padded_rank(rank);
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const Keys x{keys, stride_b, stride_h, stride_s, rows, n};
   uint16_t* v3 = static_cast<uint16_t*>(workspace);
   hipLaunchKernelGGL(factors_split_kernel, dim3(n / 32, rpad / 8, batch), dim3(256), 0, s, w, vt, rank, rpad, n, v3, sv,
                      sv_stride_b);
   const int rb = (rows + kPRows - 1) / kPRows;
-  // Five vector tiles per workgroup read K once, but leave CUs idle below 128 blocks of rows.
-  if (rtiles % 5 == 0 && static_cast<int64_t>(rb) * batch >= 128)
-    hipLaunchKernelGGL(project_kernel<5>, dim3(rb, rtiles / 5, batch), dim3(256), 0, s, x, v3, rpad, w, rank, u,
-                       u_stride_b);
-  else
-    hipLaunchKernelGGL(project_kernel<1>, dim3(rb, rtiles, batch), dim3(256), 0, s, x, v3, rpad, w, rank, u, u_stride_b);
+  const int nt = project_tiles(rtiles, static_cast<int64_t>(rb) * batch);
+  const dim3 grid(rb, (rtiles + nt - 1) / nt, batch);
+  auto go = [&](auto form) {
+    hipLaunchKernelGGL(project_kernel<decltype(form)::value>, grid, dim3(256), 0, s, x, v3, rpad, w, rank, u, u_stride_b);
+  };
+  if (nt == 1) go(std::integral_constant<int, 1>{});
+  else if (nt == 2) go(std::integral_constant<int, 2>{});
+  else if (nt == 3) go(std::integral_constant<int, 3>{});
+  else go(std::integral_constant<int, 5>{});
   return skv_check_launch(what);
 }

@@ -194,3 +194,24 @@ def test_prefill_refusals_leave_the_store(gpu):
         attn.prefill(q, k, v, None, 0)
     torch.cuda.synchronize()
     assert not cache.v_cache_cpu[0].any() and cache.prefilled_batch == 0
+
+
+@pytest.mark.parametrize("rows,R", [(600, 192), (50200, 32), (70000, 64), (50200, 72), (50200, 96), (33000, 128), (44000, 160),
+                                    (50200, 132), (50200, 160), (33000, 164), (50200, 192), (50200, 200)])
+def test_factors_forms(gpu, rows, R):
+    """Each form of the projection (1, 2, 3 and 5 tiles of 32 vectors a workgroup) with whole and partial last groups
+    and tiles, at one head; the bound of test_gram_and_factors."""
+    _say(f"factors rows={rows} R={R}")
+    n = 256 if R > 128 else 128
+    g = torch.Generator().manual_seed(rows + R)
+    k = torch.randn(1, rows, n // 128, 128, generator=g).to(torch.bfloat16)
+    vt = torch.randn(1, R, n, generator=g) / n ** 0.5
+    w = torch.rand(1, R, generator=g) * 4 + 0.5
+    u = torch.full((1, rows + 1, R), 7.0, dtype=torch.bfloat16, device=gpu)
+    sv = torch.empty(1, n // 128, 128, R, dtype=torch.bfloat16, device=gpu)
+    shadowkv.keys_factors(k.to(gpu), w.to(gpu), vt.to(gpu), u[:, :rows], sv)
+    K, V, s = k.view(rows, n).double(), vt[0].double().T, w[0].double().sqrt()
+    want = (K @ V) / s
+    lim = want.abs() * (2 ** -8 + 2 ** -20) + n * 2 ** -24 * (K.abs() @ V.abs()) / s
+    assert ((u[0, :rows].cpu().double() - want).abs() <= lim + 1e-30).all()
+    assert (u[0, rows] == 7).all(), "wrote past the rows"
