@@ -343,7 +343,7 @@ class ShadowKVCache_CPU(KVCacheBase):
         store = self.v_cache_cpu[layer_idx]
         v = new_v_cache
         if not (self.value_store == "host" and plain_eager(v) and v.dtype == store.dtype and v.stride(-1) == 1
-                and v.stride(-2) == D and 0 < n <= store.shape[2] and pb + bsz <= store.shape[0] and bsz * H <= 64
+                and v.stride(-2) == D and 0 < n <= store.shape[2] and pb + bsz <= store.shape[0]
                 and v.device == self.copy_stream.device and not torch.cuda.is_current_stream_capturing()):
             return None
         dst = store[pb:pb + bsz, :, :n]

@@ -215,3 +215,18 @@ def test_factors_forms(gpu, rows, R):
     lim = want.abs() * (2 ** -8 + 2 ** -20) + n * 2 ** -24 * (K.abs() @ V.abs()) / s
     assert ((u[0, :rows].cpu().double() - want).abs() <= lim + 1e-30).all()
     assert (u[0, rows] == 7).all(), "wrote past the rows"
+
+
+@pytest.mark.parametrize("max_length", [1400, 1480])
+def test_value_copy_of_many_rows(gpu, max_length):
+    """More than 64 (sequence, head) rows, as one transfer and row by row."""
+    B, H, ctx, D, c = 33, 2, 1400, 128, 8
+    _say(f"value copy of {B * H} rows, max={max_length}")
+    cfg = types.SimpleNamespace(num_attention_heads=H, num_key_value_heads=H, hidden_size=H * D, num_hidden_layers=1)
+    cache = ShadowKVCache_CPU(cfg, batch_size=B, max_length=max_length, device=str(gpu), sparse_budget=1024, rank=32)
+    v = torch.randn(B, H, ctx, D, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(gpu)
+    copy = cache.start_value_copy(v, 0)
+    assert copy is not None
+    copy.synchronize()
+    assert torch.equal(cache.v_cache_cpu[0][:, :, :ctx // c], v.view(B, H, ctx // c, c * D).cpu())
+    assert not cache.v_cache_cpu[0][:, :, ctx // c:].any()
