@@ -21,7 +21,8 @@
 //
 // MI355X, 122880 x 1024 keys, rank 160 (rank 64, 128, 192: factors 59, 114, 150): Gram matrix 385 us (671 TFLOP/s; conversion and fp32 product 2480),
 // factors 156 us (774 TFLOP/s issued; product, division, roundings and transposed copies 450); 3001 rows: 47
-// and 27 us against 70 and 43. Error of G against fp64 8e-8 (fp32 product: 5e-6); of U the same.
+// and 27 us against 70 and 43. Error of G against fp64 1e-7, at most 5e-7 in
+// large batches (fp32 product: 2e-5); of U the same.
 #include <algorithm>
 #include <cstdint>
 #include <type_traits>
@@ -68,11 +69,12 @@ __global__ void __launch_bounds__(kGramThreads, 2) gram_kernel(Keys x, float* __
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 31, half = lane >> 5;
-  // Share s and its tiles on one XCD (workgroup w runs on XCD w mod 8): the tiles read the same rows.
-  const int w = blockIdx.x, g8 = w / (8 * tiles), r8 = w - g8 * 8 * tiles;
-  const int share = 8 * g8 + r8 % 8, tile = r8 / 8;
-  if (share >= shares) return;  // workgroup-uniform
+  // Share s and its tiles on one XCD (workgroup w runs on XCD w mod 8): the tiles read the same rows. The next
+  // sequence's shares begin on the XCD after this one's last (batch 13 of 122880 x 1024 keys: 20.0 -> 2.8 ms).
   const int b = blockIdx.y;
+  const int w = blockIdx.x, g8 = w / (8 * tiles), r8 = w - g8 * 8 * tiles;
+  const int share = 8 * g8 + ((r8 - (b % 8) * shares) & 7), tile = r8 / 8;
+  if (share >= shares) return;  // workgroup-uniform
   int ti, tj;
   tile_of(tile, ti, tj);
   const bool diag = ti == tj;
@@ -300,11 +302,15 @@ __global__ void __launch_bounds__(256, 1) project_kernel(Keys x, const uint16_t*
 
 bool aligned(const void* p, unsigned n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
 
-// Shares of the rows: enough workgroups for the 256 CUs (one each, 128 KB of LDS), at least four stages each.
+// Shares of the rows: enough workgroups for the 256 CUs (one each, 128 KB of LDS), at least four stages each and at
+// most kShareRows rows, whatever the batch: the error of a share's fp32 sums grows with its rows (122880 x 1024 keys,
+// relative to float64: 1.0e-7 in shares of 4928 rows, 2.2e-7 of 15360, 2.2e-6 in one; torch's fp32 product 2.1e-5).
+constexpr int kShareRows = 16384;
 void gram_plan(int rows, int n, int batch, int* tiles, int* shares, int* share_rows) {
   const int nt = (n + kTile - 1) / kTile;
   *tiles = nt * (nt + 1) / 2;
-  const int want = std::max(1, std::min(256 / (*tiles * batch), (rows + 4 * kStage - 1) / (4 * kStage)));
+  const int fill = std::min(256 / (*tiles * batch), (rows + 4 * kStage - 1) / (4 * kStage));
+  const int want = std::max({1, fill, (rows + kShareRows - 1) / kShareRows});
   *share_rows = ((rows + want - 1) / want + kStage - 1) / kStage * kStage;
   *shares = (rows + *share_rows - 1) / *share_rows;
 }

@@ -230,3 +230,19 @@ def test_value_copy_of_many_rows(gpu, max_length):
     copy.synchronize()
     assert torch.equal(cache.v_cache_cpu[0][:, :, :ctx // c], v.view(B, H, ctx // c, c * D).cpu())
     assert not cache.v_cache_cpu[0][:, :, ctx // c:].any()
+
+
+@pytest.mark.parametrize("B,rows", [(11, 700), (9, 2500), (20, 100), (300, 17000)])
+def test_gram_of_large_batches(gpu, B, rows):
+    """Batches whose sequences' shares begin on another XCD each, with fewer shares than XCDs, one, and several
+    because a share is full; the bound of test_gram_and_factors, and equal sequences have equal bits."""
+    _say(f"gram of a batch of {B} x {rows}")
+    g = torch.Generator().manual_seed(rows)
+    k = torch.randn(min(B, 20), rows, 1, 128, generator=g).to(torch.bfloat16)
+    dev = k.to(gpu) if B <= 20 else k[:1].to(gpu).expand(B, rows, 1, 128)
+    gram = shadowkv.keys_gram(dev)
+    K = k[:, :, 0].double() if B <= 20 else k[:1, :, 0].double()
+    want = K.transpose(1, 2) @ K
+    lim = rows * 2 ** -24 * (K.abs().transpose(1, 2) @ K.abs()) + 1e-30
+    assert ((gram[:len(K)].cpu().double() - want).abs() <= lim).all()
+    assert B <= 20 or (gram == gram[:1]).all()

@@ -136,3 +136,16 @@ def test_fetch_workgroups_follow_the_environment(env, want):
     clean = {k: v for k, v in os.environ.items() if k not in ("SKV_FETCH_WGS", "SKV_FUSED_FETCH_WGS")}
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100, env={**clean, **env})
     assert r.returncode == 0 and r.stdout.strip() == want, (r.stdout, r.stderr)
+
+
+@pytest.mark.parametrize("batch,rows,heads", [(1, 122880, 8), (4, 122880, 8), (13, 122880, 8), (64, 122881, 8),
+                                              (300, 60000, 1), (64, 262144, 2), (26, 100, 8)])
+def test_gram_shares_hold_at_most_16384_rows(batch, rows, heads):
+    """The rows that skv_keys_gram sums in one fp32 chain, read off its workspace (256 x 256 fp32 tiles of the lower
+    triangle per share): bounded whatever the batch."""
+    nt = (heads * 128 + 255) // 256
+    tile_bytes = nt * (nt + 1) // 2 * 256 * 256 * 4
+    nbytes = _lib.lib().skv_keys_gram_workspace_bytes(batch, rows, heads)
+    assert nbytes % (batch * tile_bytes) == 0
+    shares = nbytes // (batch * tile_bytes)
+    assert shares * 16384 >= rows and shares <= max(256 // (batch * nt * (nt + 1) // 2), -(-rows // 16384), 1)
