@@ -268,7 +268,8 @@ class ShadowKVCache_CPU(KVCacheBase):
 
     def _keys_in_place(self, k: torch.Tensor):
         """The keys as [b, ctx, H, 128] without a copy, where the factor kernels read them (bf16, 16-byte
-        aligned rows, up to 1024 columns, a rank that is a multiple of 4), else None."""
+        aligned rows, up to 1024 columns, a rank that is a multiple of 4, a batch that a grid dimension holds),
+        else None."""
         H, D = self.num_key_value_heads, self.head_dim
         if k.dim() == 4 and k.shape[1] == H and k.shape[1] <= 32 and k.shape[3] == D:
             k = k.transpose(1, 2)
@@ -279,7 +280,8 @@ class ShadowKVCache_CPU(KVCacheBase):
         ok = (plain_eager(k) and k.dtype == torch.bfloat16 and self.dtype == torch.bfloat16 and D == 128
               and 64 <= H * D <= shadowkv.KEYS_MAX_COLUMNS and self.rank % 4 == 0 and self.rank <= H * D
               and k.numel() > 0 and k.device == self.U.device and k.stride(3) == 1 and k.data_ptr() % 16 == 0
-              and not any(s % 8 for s in k.stride()[:3]) and k.shape[0] <= 64 and shadowkv.sym_eig_runs_on(k.device))
+              and not any(s % 8 for s in k.stride()[:3]) and k.shape[0] <= 65535
+              and shadowkv.sym_eig_runs_on(k.device))
         return k if ok else None
 
     def _alloc_landmarks(self, n: int):

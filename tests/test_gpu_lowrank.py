@@ -246,3 +246,19 @@ def test_gram_of_large_batches(gpu, B, rows):
     lim = rows * 2 ** -24 * (K.abs().transpose(1, 2) @ K.abs()) + 1e-30
     assert ((gram[:len(K)].cpu().double() - want).abs() <= lim).all()
     assert B <= 20 or (gram == gram[:1]).all()
+
+
+def test_get_svd_of_a_large_batch(gpu, monkeypatch):
+    """More than 64 sequences at once: by the kernels, the same factors as each sequence's own."""
+    B, ctx, R = 67, 300, 32
+    _say(f"get_svd of {B} sequences")
+    k = torch.randn(B, 1, ctx, 128, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16).to(gpu)
+    cfg = types.SimpleNamespace(num_attention_heads=1, num_key_value_heads=1, hidden_size=128, num_hidden_layers=1)
+    make = dict(max_length=ctx, device=str(gpu), sparse_budget=64, rank=R, value_store="device")
+    monkeypatch.setattr(kv, "low_rank_factors", lambda *a: pytest.fail("not by the kernels"))
+    cache = ShadowKVCache_CPU(cfg, batch_size=B, **make)
+    cache.get_svd(k, 0)
+    for b in (0, 8, 66):
+        one = ShadowKVCache_CPU(cfg, batch_size=1, **make)
+        one.get_svd(k[b:b + 1], 0)
+        assert torch.equal(cache.U[0][b], one.U[0][0]) and torch.equal(cache.SV[0][b], one.SV[0][0])
