@@ -243,7 +243,8 @@ class ShadowKVCache_CPU(KVCacheBase):
         self._require_device(new_k_cache)
         H, D, R = self.num_key_value_heads, self.head_dim, self.rank
         if new_k_cache.shape[1] <= 32:
-            bsz, ctx = new_k_cache.shape[0], new_k_cache.shape[-2]
+            bsz = new_k_cache.shape[0]
+            ctx = new_k_cache.numel() // max(1, bsz * H * D)  # (whatever its heads: H * D columns are made of it)
         else:
             bsz, ctx = new_k_cache.shape[:2]
         if layer_idx == 0 and self.prefilled_batch == 0:

@@ -262,3 +262,19 @@ def test_get_svd_of_a_large_batch(gpu, monkeypatch):
         one = ShadowKVCache_CPU(cfg, batch_size=1, **make)
         one.get_svd(k[b:b + 1], 0)
         assert torch.equal(cache.U[0][b], one.U[0][0]) and torch.equal(cache.SV[0][b], one.SV[0][0])
+
+
+def test_get_svd_of_regrouped_heads(gpu):
+    """Keys by head whose heads are not the cache's: taken as rows of H * D columns, as their transpose gives them."""
+    _say("get_svd of regrouped heads")
+    H, ctx, R = 4, 300, 32
+    cfg = types.SimpleNamespace(num_attention_heads=H, num_key_value_heads=H, hidden_size=H * 128, num_hidden_layers=1)
+    make = dict(batch_size=1, max_length=ctx, device=str(gpu), sparse_budget=64, rank=R, value_store="device")
+    for heads, rows in ((2, 2 * ctx), (8, ctx // 2)):
+        k = torch.randn(1, heads, rows, 128, generator=torch.Generator().manual_seed(heads)).to(torch.bfloat16).to(gpu)
+        got, want = ShadowKVCache_CPU(cfg, **make), ShadowKVCache_CPU(cfg, **make)
+        got.get_svd(k, 0)
+        want.get_svd(k.transpose(1, 2).reshape(1, ctx, H * 128), 0)
+        assert got.U.shape == want.U.shape == (1, 1, ctx, R)
+        a, b = (torch.einsum("bcr,bhdr->bchd", c.U[0].float().cpu(), c.SV[0].float().cpu()) for c in (got, want))
+        assert (a - b).norm() <= 8e-3 * b.norm()  # two roundings to bf16 of either route's factors
