@@ -58,16 +58,6 @@ struct EigenArgs {
   int batch;
 };
 
-template <int C, int CTRL>
-__device__ __forceinline__ void fold(float* v, bool upper) {
-#pragma unroll
-  for (int j = 0; j < C / 2; ++j) {
-    const float keep = upper ? v[C / 2 + j] : v[j];
-    const float send = upper ? v[j] : v[C / 2 + j];
-    v[j] = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(send), CTRL, 0xf, 0xf, false));
-  }
-}
-
 // Element idx of a vector held as x[r] = element 64 r + lane, idx wave-uniform with idx / 64 in [LO, HI].
 template <int LO, int HI, class Col>
 __device__ __forceinline__ float pick(const Col& x, int idx) {
@@ -155,10 +145,10 @@ struct Reduction {
         f[s] = p;
         f[kCols + s] = mine ? c : 0.f;
       });
-      fold<16, 0x140>(f, lane & 8);
-      fold<8, 0x141>(f, lane & 4);
-      fold<4, 0x1B>(f, lane & 2);
-      fold<2, 0xB1>(f, lane & 1);
+      skv::fold<16, 0x140>(f, lane & 8);
+      skv::fold<8, 0x141>(f, lane & 4);
+      skv::fold<4, 0x1B>(f, lane & 2);
+      skv::fold<2, 0xB1>(f, lane & 1);
       {
         const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(f[0]), __float_as_uint(f[0]), false, false);
         f[0] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
@@ -249,10 +239,12 @@ struct Reduction {
   }
 };
 
-// (One wave per SIMD with up to 512 registers: 8 columns of 1024 rows are 128 of them; two waves of
-// 4 columns would do the redundant vector work twice.)
+// (Compiled for one wave per SIMD, so that the 8 columns, 128 registers at 1024 rows, stay in registers with all that
+// the steps hold; two waves of 4 columns would do the redundant vector work twice. At 232 registers two
+// workgroups still fit on a CU, 64 on an XCD.)
 // A workgroup takes its part by its order of arrival on its XCD: problem b runs on XCD b, its
-// 2 NR workgroups one per CU on an idle device (a request for LDS that forces it changes nothing).
+// 2 NR workgroups spread over the CUs of an idle device by the dispatcher (a request for LDS that forces one per CU
+// changes nothing).
 template <int NR>
 __global__ void __launch_bounds__(kWgWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 tridiag_kernel(EigenArgs g) {

@@ -24,6 +24,7 @@
 
 #include "rope_math.h"
 #include "skv_common.h"
+#include "wave_reduce.h"
 
 namespace {
 
@@ -79,19 +80,6 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), c, false);
 }
 
-// One transpose-reduce step over the lane bit that the DPP pattern CTRL flips: lanes with the
-// bit set keep the upper half of their C values, the others the lower half, and each adds the
-// partner's copy of the half it keeps.
-template <int C, int CTRL>
-__device__ __forceinline__ void fold(float* v, bool upper) {
-#pragma unroll
-  for (int j = 0; j < C / 2; ++j) {
-    const float keep = upper ? v[C / 2 + j] : v[j];
-    const float send = upper ? v[j] : v[C / 2 + j];
-    v[j] = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(send), CTRL, 0xf, 0xf, false));
-  }
-}
-
 // bf16 pair of silu(g) * u from the bf16 pairs g2, u2 (element 0 in the low half), with the
 // arithmetic and roundings of the SiLU-and-mul kernel (skv::silu_mul, then one bf16 rounding).
 __device__ __forceinline__ uint32_t silu_mul2(uint32_t g2, uint32_t u2) {
@@ -110,7 +98,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64) linear_kernel(const uint16_t* 
                                                                uint16_t* __restrict__ y, int64_t ys, int M, int N,
                                                                int K, RopeEpi re) {
   constexpr int V = R * MP;  // partial sums per lane
-  static_assert(V >= 16 && V <= 64 && (V & (V - 1)) == 0, "R * MP must be 16, 32 or 64");
+  static_assert(V == 16 || V == 32, "R * MP must be 16 or 32");
   static_assert(!(kGated && kAct) && (!kAct || R % 2 == 0), "gate/up pairs need an even row count");
   static_assert(kRope == kNoRope || (!kGated && !kAct && R % 2 == 0 && kHeadDim % R == 0),
                 "the RoPE epilogue takes whole rotation pairs of one head per workgroup");
@@ -224,10 +212,10 @@ __global__ void __launch_bounds__(kMaxWaves * 64) linear_kernel(const uint16_t* 
 #pragma unroll
     for (int m = 0; m < MP; ++m) v[r * MP + m] = acc[r][m];
   const int p = lane & 15;
-  fold<V, 0x140>(v, p & 8);
-  fold<V / 2, 0x141>(v, p & 4);
-  fold<V / 4, 0x1B>(v, p & 2);
-  fold<V / 8, 0xB1>(v, p & 1);
+  skv::fold<V, 0x140>(v, p & 8);
+  skv::fold<V / 2, 0x141>(v, p & 4);
+  skv::fold<V / 4, 0x1B>(v, p & 2);
+  skv::fold<V / 8, 0xB1>(v, p & 1);
   constexpr int kPer = V / 16;
   float* dst = red + (wave * 4 + (lane >> 4)) * V + p * kPer;
 #pragma unroll
@@ -279,8 +267,8 @@ __global__ void __launch_bounds__(kMaxWaves * 64) linear_kernel(const uint16_t* 
 
 
 // The matrix-core form, for 5 to 16 token rows. Bound: the weight stream from HBM. The dot2 form
-// above needs R * MP accumulators and re-reads x once per R weight rows, so at 9..16 rows, where
-// registers leave R = 2, its x traffic from the L2 is eight times the weight stream and bounds it.
+// above needs R * MP accumulators and re-reads x once per R weight rows: for 9..16 rows registers would
+// leave R = 2, and its x traffic from the L2, eight times the weight stream, bounded it.
 // Here a workgroup owns 16 weight rows (one 16x16 MFMA tile; 8 of a small weight, for twice the
 // workgroups) and its waves split K into 128-element
 // blocks (wave w takes blocks w, w + NW, ...). A wave reads its block of the weight and x rows with
@@ -445,7 +433,7 @@ __global__ void __launch_bounds__(NW * 64) linear_mfma_kernel(const uint16_t* __
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-int g_waves_override = -1;  // SKV_LINEAR_WAVES, read once
+int g_waves_override = -1;  // SKV_LINEAR_WAVES (the dot2 form's waves), read once
 
 template <int R, int MP, bool kGated, bool kAct = false, int kRope = kNoRope>
 void launch(const uint16_t* x, int64_t xs, const uint16_t* w, int64_t ws, uint16_t* y, int64_t ys, int M, int N, int K,

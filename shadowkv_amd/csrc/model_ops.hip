@@ -34,7 +34,8 @@ __device__ __forceinline__ u32x4 pack8(const float* f) {
 // One workgroup per row; each thread owns 8-element vectors strided by the workgroup. Bound by
 // latency (8 KB rows, a few workgroups): one trip to memory, the weights requested with the row and
 // not after the reduction, and one vector per thread up to 4096 elements.
-constexpr int kNormThreads = 512;
+constexpr int kNormThreads = 512, kNormVecs = 2;
+constexpr int kNormMaxHidden = 8 * kNormVecs * kNormThreads;
 
 template <bool kResidual>
 __global__ void __launch_bounds__(kNormThreads) rmsnorm_kernel(const uint16_t* __restrict__ x, int64_t xs,
@@ -42,7 +43,7 @@ __global__ void __launch_bounds__(kNormThreads) rmsnorm_kernel(const uint16_t* _
                                                                uint16_t* __restrict__ ro, int64_t ros,
                                                                const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
                                                                int64_t os, int hidden, float eps) {
-  constexpr int kMaxVec = 2;  // hidden <= 2 * 8 * 512 = 8192
+  constexpr int kMaxVec = kNormVecs;
   __shared__ float part[kNormThreads / 64];
   const int row = blockIdx.x;
   const int nv = hidden / 8;
@@ -183,8 +184,8 @@ extern "C" int skv_rmsnorm(const uint16_t* x, int64_t x_stride, const uint16_t* 
     skv_set_error("%s: null pointer", what);
     return SKV_EINVAL;
   }
-  if (rows < 1 || hidden < 8 || hidden % 8 || hidden > 8 * 4 * kThreads) {
-    skv_set_error("%s: rows=%d hidden=%d (hidden a multiple of 8 up to %d)", what, rows, hidden, 8 * 4 * kThreads);
+  if (rows < 1 || hidden < 8 || hidden % 8 || hidden > kNormMaxHidden) {
+    skv_set_error("%s: rows=%d hidden=%d (hidden a multiple of 8 up to %d)", what, rows, hidden, kNormMaxHidden);
     return SKV_EUNSUPPORTED;
   }
   if (!aligned16(x) || !aligned16(weight) || !aligned16(out) || x_stride % 8 || out_stride % 8 ||

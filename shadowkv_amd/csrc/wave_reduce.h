@@ -1,4 +1,4 @@
-// Reduce-scatter of M per-lane partial sums over an aligned group of 16 lanes.
+// Reduce-scatters of per-lane partial sums: of M over an aligned group of 16 lanes (below), and one DPP step of one (fold).
 //
 // Each of the 16 lanes holds v[0..M) (partial dot products over its slice of the head
 // dimension). After log2(M) halving exchanges (xor 8, 4, ...) every lane holds the group
@@ -56,6 +56,19 @@ template <int M>
 __device__ __forceinline__ float reduce_scatter16(float* v, int li) {
   static_assert(M >= 1 && M <= 16 && (M & (M - 1)) == 0, "M must be a power of two <= 16");
   return ReduceScatter16<M, 8>::run(v, li);
+}
+
+// One transpose-reduce step over the lane bit that the DPP pattern CTRL flips: lanes with the
+// bit set keep the upper half of their C values, the others the lower half, and each adds the
+// partner's copy of the half it keeps.
+template <int C, int CTRL>
+__device__ __forceinline__ void fold(float* v, bool upper) {
+#pragma unroll
+  for (int j = 0; j < C / 2; ++j) {
+    const float keep = upper ? v[C / 2 + j] : v[j];
+    const float send = upper ? v[j] : v[C / 2 + j];
+    v[j] = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(send), CTRL, 0xf, 0xf, false));
+  }
 }
 
 }  // namespace skv

@@ -1,9 +1,11 @@
 """ShadowKV attention handler (reference: models/attention/shadow.py:6-50).
 
-decode() keeps the reference's order of operations and its two-stream overlap:
-RoPE -> append the new token -> select chunks (score, top-k, reorder) -> [copy stream: value
-fetch from host] || [current stream: key compaction + low-rank rebuild + RoPE] -> join ->
-sparse attention. The attention is the gfx950 split-L decode kernel in place of
+decode() keeps the reference's order of operations: RoPE -> append the new token -> select chunks
+(score, top-k, reorder) -> value fetch from host beside the low-rank key rebuild + RoPE -> sparse
+attention. A cache in its default setting takes the fetch and the rebuild as one launch on the current
+stream, after a selection that moves the cached chunks itself; otherwise, and in decode_begin() /
+decode_end(), they are the reference's two streams: [copy stream: value fetch] || [current stream: key
+compaction + rebuild] -> join. The attention is the gfx950 split-L decode kernel in place of
 flash_attn_with_kvcache; prefill attention is the gfx950 prompt attention kernel (fp32 torch operations
 where that kernel does not apply).
 """
