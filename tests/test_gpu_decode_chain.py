@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from shadowkv_amd.decode_model import synthesize_state
-from shadowkv_amd.models.attention import ShadowAttention
+from shadowkv_amd.models.attention import ShadowAttention, shadow
 from shadowkv_amd.models.kvcache import ShadowKVCache_CPU
 from shadowkv_amd.models.tensor_op import apply_rotary_pos_emb_cuda, build_cos_sin_cache, build_glm_cos_sin_cache
 
@@ -24,7 +24,7 @@ def _say(msg):
     (3, 3, 1, 9001, 2048, 16, "host", False), (2, 2, 4, 40000, 16384, 8, "host", False),
     (2, 8, 4, 6000, 1024, 8, "device", False), (1, 2, 16, 20011, 2048, 16, "device", True),
     (16, 8, 4, 6000, 4096, 8, "host", False)])
-def test_decode_equals_begin_and_end(gpu, B, H, G, ctx, budget, chunk, store, glm):
+def test_decode_equals_begin_and_end(gpu, monkeypatch, B, H, G, ctx, budget, chunk, store, glm):
     _say(f"decode chain B={B} H={H} G={G} ctx={ctx} budget={budget} chunk={chunk} {store} glm={glm}")
     D, steps = 128, 4
     table = (build_glm_cos_sin_cache(ctx + 64, 10000.0, device=gpu) if glm
@@ -48,6 +48,9 @@ def test_decode_equals_begin_and_end(gpu, B, H, G, ctx, budget, chunk, store, gl
                                   chunk_size=chunk, rank=64, max_decode_len=steps, value_store=store)
         synthesize_state(cache, ctx, seed=7, cos_sin=table)
         attn = ShadowAttention(cache, G, D, H * G * D, rope, None, table)
+        if store == "host" and budget > 8192:  # (not the chain that decode() takes by itself at this width)
+            monkeypatch.setitem(shadow.JOINED_MAX_BUDGET, store, budget)
+        assert attn._joined(cache)
         outs = []
         for i in range(steps):
             pos = torch.full((1, 1, 1), ctx + i, dtype=torch.int64, device=gpu)
@@ -196,7 +199,6 @@ def test_wide_selections_keep_the_two_streams(gpu, monkeypatch, store, budget, j
     """A selection too wide for its rows' workgroups to move the hits: the two-stream chain, with the bits of
     the joined one."""
     _say(f"decode chain {store} budget={budget}")
-    from shadowkv_amd.models.attention import shadow
     ctx, chunk = 60000, 16
     cfg = types.SimpleNamespace(num_attention_heads=8, num_key_value_heads=2, hidden_size=1024, num_hidden_layers=1)
     table = build_cos_sin_cache(ctx + 8, 500000.0, 128, device=gpu)

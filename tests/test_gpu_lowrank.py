@@ -88,7 +88,10 @@ def test_get_svd_routes(gpu, form, monkeypatch):
         real = ShadowKVCache_CPU._keys_in_place
         monkeypatch.setattr(ShadowKVCache_CPU, "_keys_in_place",
                             lambda self, x: None if force else (taken.append(real(self, x)) or taken[-1]))
-        cache.get_svd(arg, 0)
+        with monkeypatch.context() as m:
+            if not force and form != "odd":  # (the kernels' own factors, and a verdict that takes them)
+                m.setattr(kv, "low_rank_factors", lambda *a: pytest.fail("the kernels' factors were not taken"))
+            cache.get_svd(arg, 0)
         monkeypatch.setattr(ShadowKVCache_CPU, "_keys_in_place", real)
         if not force:
             assert (taken[0] is None) == (form == "odd")
@@ -97,6 +100,32 @@ def test_get_svd_routes(gpu, form, monkeypatch):
     assert diff < 4e-3, diff  # two bf16 roundings of the same fp32 factors, up to their signs
     err = (rec[0].reshape(B, ctx, -1) - k.double()).norm() / k.double().norm()
     assert err < 0.08  # the noise outside rank 64
+
+
+def test_get_svd_after_a_refused_verdict(gpu, monkeypatch):
+    """Eigenpairs that do not hold up, whose factors are written before the host reads the verdict: replaced by the
+    torch operations' factors."""
+    _say("get_svd after a refused verdict")
+    H, ctx, R = 2, 700, 64
+    k = torch.randn(1, H, ctx, 128, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).to(gpu)
+    cfg = types.SimpleNamespace(num_attention_heads=H, num_key_value_heads=H, hidden_size=H * 128, num_hidden_layers=1)
+    make = dict(batch_size=1, max_length=ctx, device=str(gpu), sparse_budget=64, rank=R, value_store="device")
+    want = ShadowKVCache_CPU(cfg, **make)
+    with monkeypatch.context() as m:
+        m.setattr(ShadowKVCache_CPU, "_keys_in_place", lambda self, x: None)
+        want.get_svd(k, 0)
+    got = ShadowKVCache_CPU(cfg, **make)
+    real, calls = kv._top_eigenpairs, []
+
+    def refuse_first(gram, rank):
+        w, vt, ok = real(gram, rank)
+        calls.append(bool(ok))
+        return (w, vt, ok) if len(calls) > 1 else (w.fill_(float("nan")), vt.fill_(3.0), torch.zeros_like(ok))
+
+    monkeypatch.setattr(kv, "_top_eigenpairs", refuse_first)
+    got.get_svd(k, 0)
+    assert calls == [True, True]
+    assert torch.equal(got.U, want.U) and torch.equal(got.SV, want.SV)
 
 
 @pytest.mark.parametrize("ctx,max_length,B,first", [(1400, 1400, 2, 2), (1403, 2048, 2, 1), (1800, 4096, 3, 2)])

@@ -25,9 +25,9 @@ def _exact(q, k, v):
 
 
 # Lengths around the 64-key tiles and the 32- and 128-query blocks; (batch, kv head) rows that divide
-# among the 8 XCDs, that the XCDs divide among, and neither.
+# among the 8 XCDs (once and several times), that the XCDs divide among, and neither.
 @pytest.mark.parametrize("L", [1, 31, 64, 65, 127, 129, 300])
-@pytest.mark.parametrize("B,Hq,H", [(1, 8, 8), (2, 4, 1), (1, 6, 3), (3, 16, 1)])
+@pytest.mark.parametrize("B,Hq,H", [(1, 8, 8), (2, 4, 1), (1, 6, 3), (3, 16, 1), (2, 16, 8), (3, 16, 8), (1, 5, 5)])
 def test_prefill_attn_edges(gpu, B, Hq, H, L):
     """Bound: one bf16 rounding (2^-8) of the value; fp32 scores of magnitude <= ~20 err by 20 * 2^-22
     relative in a probability, so 1e-4 of the largest value is ample."""
