@@ -17,6 +17,7 @@ sparse_attn_decode) expose the fused kernels used by the decode path.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -396,6 +397,7 @@ def _rebuild_geometry(u, sv, position_ids, cnts, cos_sin, cache, sparse_start, c
     return u_sb, u_sh, u_sr, u_rows, sv_sb, sv_sh, sv_sn, mode, rank
 
 
+@functools.lru_cache(maxsize=64)
 def fetch_workgroups_alone(rows: int, num_chunks: int) -> int:
     """The fetch workgroups of a fetch_misses_rebuild_k_rope launch from pinned host memory that no other work
     runs beside, for rows rows of num_chunks slots: the library's count, or SKV_FUSED_FETCH_WGS or
@@ -1075,11 +1077,12 @@ SYM_EIG_MAX_N = 1024
 SYM_EIG_MAX_BATCH = 8
 
 
-def sym_eig_runs_on(device) -> bool:
+@functools.lru_cache(maxsize=64)
+def sym_eig_runs_on(device_index: int) -> bool:
     """Whether sym_eig_top's problems find the XCDs that they run on: a whole MI355X (8 XCDs of 32 CUs). In a
     partition of one, XCDs are missing, and which ids the others have is not stated: problems of an absent id
     would never be solved (their status stays 0), and every caller would pay for the attempt."""
-    return torch.cuda.get_device_properties(device).multi_processor_count >= 8 * 32
+    return torch.cuda.get_device_properties(device_index).multi_processor_count >= 8 * 32
 
 
 def sym_eig_top(a, rank):

@@ -56,7 +56,11 @@ def causal_attention_fp32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, blo
 def _unreplaced(obj, steps: dict) -> bool:
     """Whether obj's methods named in steps are the functions that steps holds: not another class's, not a
     subclass's and not the instance's own."""
-    return all(getattr(type(obj), n, None) is f for n, f in steps.items()) and steps.keys().isdisjoint(vars(obj))
+    cls = type(obj)
+    for name, function in steps.items():
+        if getattr(cls, name, None) is not function or name in obj.__dict__:
+            return False
+    return True
 
 
 # Selected tokens (sparse_budget) up to which the joined chain is taken, by value store: its selection moves both

@@ -45,7 +45,7 @@ def _top_eigenpairs(gram: torch.Tensor, rank: int):
     largest eigenvalue, orthogonality 1 to 2.3e-6; the kernel's own: 0.8 to 1.8e-7 and 0.2 to 0.9e-6)."""
     b, n, _ = gram.shape
     if not (plain_eager(gram) and gram.dtype == torch.float32 and 64 <= n <= shadowkv.SYM_EIG_MAX_N and 1 <= rank <= n
-            and b > 0 and shadowkv.sym_eig_runs_on(gram.device)) or torch.cuda.is_current_stream_capturing():
+            and b > 0 and shadowkv.sym_eig_runs_on(gram.device.index)) or torch.cuda.is_current_stream_capturing():
         return None
     ws, vts, good = [], [], []
     with torch.cuda.device(gram.device):
@@ -282,7 +282,7 @@ class ShadowKVCache_CPU(KVCacheBase):
               and 64 <= H * D <= shadowkv.KEYS_MAX_COLUMNS and self.rank % 4 == 0 and self.rank <= H * D
               and k.numel() > 0 and k.device == self.U.device and k.stride(3) == 1 and k.data_ptr() % 16 == 0
               and not any(s % 8 for s in k.stride()[:3]) and k.shape[0] <= 65535
-              and shadowkv.sym_eig_runs_on(k.device))
+              and shadowkv.sym_eig_runs_on(k.device.index))
         return k if ok else None
 
     def _alloc_landmarks(self, n: int):

@@ -148,13 +148,15 @@ def test_captured_call(gpu):
         torch.cuda.synchronize()
 
 
-def test_part_of_a_device_takes_eigh(gpu, monkeypatch):
+def test_part_of_a_device_takes_eigh(gpu, monkeypatch, request):
     """A device that reports fewer CUs than the XCDs of a whole one have: no attempt, eigh's factors."""
     _say("eigen: part of a device")
     g = torch.Generator().manual_seed(4)
     k = torch.randn(1, 300, 128, generator=g).to(gpu)
     u, svt = kv.low_rank_factors(k, 8)
     monkeypatch.setattr(torch.cuda, "get_device_properties", lambda d: types.SimpleNamespace(multi_processor_count=128))
+    shadowkv.sym_eig_runs_on.cache_clear()
+    request.addfinalizer(shadowkv.sym_eig_runs_on.cache_clear)
     monkeypatch.setattr(shadowkv, "sym_eig_top", lambda *a: pytest.fail("attempted"))
     assert kv._top_eigenpairs(torch.matmul(k.transpose(1, 2).contiguous(), k), 8) is None
     cfg = types.SimpleNamespace(num_attention_heads=2, num_key_value_heads=1, hidden_size=256, num_hidden_layers=1)
